@@ -234,6 +234,44 @@ def test_gemm_split_block_ranges(dev, qt, zq, case, rows, k, m, plain_what, min_
         dev.free_resident(res)
 
 
+# The wide fp6 GEMM (q4_1 / q4_k, 128 tokens x 192 rows per workgroup) where the
+# host picks it: at least 7/8 of the CUs of its rounds busy.  It walks block pairs
+# in turns of three stages (three buffers), so every remainder of the stages by
+# three, odd nb, a last row tile of one row and a last token tile of one
+# token; and two rounds of whole tiles (m = 896: exactly 7/8).
+WIDE = [(synth.Q4_1, zd.Q4_1, 56 * 192 + 1, k, 385) for k in (1536, 1568, 1632, 1664)] + \
+       [(synth.Q4_K, zd.Q4_K, 56 * 192 + 1, 1792, 511), (synth.Q4_K, zd.Q4_K, 12288, 1536, 896)]
+
+
+@pytest.mark.parametrize("qt,zq,rows,k,m", WIDE, ids=[f"{GEMM_QUANT_IDS[c[0]]}-{c[2]}x{c[3]}-m{c[4]}" for c in WIDE])
+def test_gemm_wide(dev, qt, zq, rows, k, m):
+    _say(f"gemm wide type={qt} rows={rows} k={k} m={m}")
+    rb = synth.row_bytes(qt, k)
+    w = synth.weights(qt, rows, k, seed=rows + k + m)
+    xs = synth.activation(k + m, m * k)
+    res = dev.upload_resident(w)
+    x_dev = dev.dev_malloc(xs.nbytes)
+    out_dev = dev.dev_malloc(m * rows * 4)
+    try:
+        dev.dev_upload(x_dev, xs)
+        log = _route(dev, res, zq, rows, k, m, x_dev, out_dev)
+        gemm = [r for r in log if r["what"].startswith("gemm")]
+        assert [(r["what"], r["block"], r["grid_x"], r["grid_y"]) for r in gemm] == \
+            [("gemm wide", 768, (rows + 191) // 192, (m + 127) // 128)]
+        out = np.zeros(m * rows, np.float32)
+        dev.dev_download(out, out_dev)
+        got = out.reshape(m, rows)
+        # f32 sums of nb <= 56 block terms, each within a few roundings: well below 1e-6
+        for r0, r1 in ((0, 64), (rows // 2, rows // 2 + 32), (rows - 48, rows)):
+            want = oracle.matmul_int(qt, w[r0 * rb:r1 * rb], k, r1 - r0, m, xs)
+            assert rel_l2(got[:, r0:r1], want) <= 1e-6, (r0, r1)
+            assert rel_l2(got[-1, r0:r1], want.reshape(m, r1 - r0)[-1]) <= 1e-6, (r0, r1)
+    finally:
+        dev.dev_free(x_dev)
+        dev.dev_free(out_dev)
+        dev.free_resident(res)
+
+
 def test_gemm_config4_rows_subset(dev):
     """configs[4] at full size (12288 x 4096 Q4_0 x 512 tokens); rows checked
     against the oracle on a slice of the weight (a GEMM row depends only on its

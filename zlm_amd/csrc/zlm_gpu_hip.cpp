@@ -201,6 +201,9 @@ struct zlm_device {
     hipFunction_t gemm_q8_0 = nullptr;
     hipFunction_t gemm_q4_1_k2 = nullptr;
     hipFunction_t gemm_q4_k_k2 = nullptr;
+    // the wide fp6 GEMM (q4_1 / q4_k; 128-token x 192-row tiles, 12 waves) and its activations
+    hipFunction_t quantize_fp6 = nullptr;
+    hipFunction_t gemm_wide = nullptr;
     hipFunction_t qk_norm_rope_kv = nullptr;
     hipFunction_t attn_partial = nullptr;
     hipFunction_t attn_combine = nullptr;
@@ -341,6 +344,8 @@ bool load_kernels(zlm_device* d) {
                 {&d->gemm_q8_0_k2, "zlm_gemm_q8_0_q8_k2"},
                 {&d->gemm_q4_1_k2, "zlm_gemm_q4_1_q8_k2"},
                 {&d->gemm_q4_k_k2, "zlm_gemm_q4_k_q8_k2"},
+                {&d->quantize_fp6, "zlm_quantize_fp6_tiled"},
+                {&d->gemm_wide, "zlm_gemm_wide"},
                 {&d->gemm_small_q4_0, "zlm_gemm_small_q4_0_q8"},
                 {&d->gemm_small_q8_0, "zlm_gemm_small_q8_0_q8"},
                 {&d->gemm_small_q4_1, "zlm_gemm_small_q4_1_q8"},
@@ -1340,7 +1345,8 @@ double now_ns() {
 // waves per workgroup for q4_0 / q8_0, 8 for q4_1 / q4_k; one workgroup per
 // 32-row x 32-token tile); beyond it whichever of that kernel and the
 // 128 x 64 tiled int GEMM (each tile's blocks split over four or two wave
-// groups, or not) the cost model below predicts faster.
+// groups, or not) the cost model below predicts faster, or for q4_1 / q4_k the
+// wide fp6 GEMM where its rounds fill the chip.
 constexpr size_t kGemmGemvM = 2;
 constexpr size_t kGemmSmallM = 32;
 
@@ -1386,6 +1392,26 @@ double gemm_tiled_us(const QuantInfo* qi, size_t rows, size_t m, size_t nb, int 
         c = n == 2 ? 0.475 : n == 3 ? 0.67 : 0.22 * dn;
     }
     return 3.0 + c * static_cast<double>(nb);
+}
+
+// - The wide fp6 kernel (q4_1, q4_k): rounds of one 128-token x 192-row
+//   workgroup per CU, 6 us + 0.6 us per block and round with its quantizer
+//   (4.5 us of them at 512 tokens, which the tiled prediction leaves out).  Measured
+//   on q4_k, tiled and wide: 12288 x 4096 x 512 91 and 83 us, x 1999 340 and 317;
+//   15360 x 3840 x 384 84 and 76, x 1999 396 and 370.  It has no smaller tile for
+//   what is left over, so where its last round is emptier the tiled kernels take
+//   over (15360 x 3840 x 512, 320 workgroups: 107 and 139); the line is seven
+//   eighths of all rounds' CUs, the range it was measured on.
+//   Rows longer than kGemmWideMaxNb blocks keep to the other kernels (the wide
+//   kernel's offsets are 32-bit).
+constexpr uint64_t kGemmWideMaxNb = 1u << 18;
+
+bool gemm_wide_pays(const QuantInfo* qi, size_t rows, size_t m, size_t nb, int cus, double tiled_us) {
+    if (!gemm_has_min(qi->type) || nb > kGemmWideMaxNb) return false;
+    const uint64_t c = static_cast<uint64_t>(cus);
+    const uint64_t wgs = static_cast<uint64_t>((rows + 191) / 192) * static_cast<uint64_t>((m + 127) / 128);
+    const uint64_t n = (wgs + c - 1) / c;
+    return 8 * wgs >= 7 * n * c && 6.0 + 0.6 * static_cast<double>(n * nb) < tiled_us;
 }
 
 bool gemm_supported(uint32_t type) {
@@ -1495,10 +1521,16 @@ bool enqueue_gemm(zlm_device* d, zlm_resident* r, uint32_t quant, size_t rows, s
     if (!ensure_gemm_tiles(d, r, qi, nb)) return false;
     if (r->gemm_rt * 32 < rows) return fail(d, "GEMM tiles too short");
     const bool with_min = gemm_has_min(qi->type);
+    int split = 1;
+    const double tiled_us = gemm_tiled_us(qi, rows, m, nb, d->cus, &split);
+    const bool small = m <= kGemmSmallM || gemm_small_us(qi, rows, m, nb, d->cus) < tiled_us;
+    const bool wide = !small && gemm_wide_pays(qi, rows, m, nb, d->cus, tiled_us);
     const uint64_t mt = (static_cast<uint64_t>(m) + 31) / 32;
+    // the wide kernel's activations: records of 128 tokens and two blocks
+    const uint64_t gt = (static_cast<uint64_t>(m) + 127) / 128, records = gt * ((nb + 1) / 2);
     const uint64_t qbytes = mt * 32 * k;  // a multiple of 1024
     const uint64_t fbytes = mt * 32 * nb * 4;
-    const uint64_t need = qbytes + fbytes * (with_min ? 2 : 1);
+    const uint64_t need = wide ? records * 14336 : qbytes + fbytes * (with_min ? 2 : 1);
     if (need > d->q_scratch_cap && !may_replace_scratch(d, kUsesGemm, "the GEMM activation scratch")) return false;
     if (!ensure_bytes(d, d->q_scratch, d->q_scratch_cap, need)) return false;
     if (d->capturing) d->capture_uses |= kUsesGemm;
@@ -1507,6 +1539,16 @@ bool enqueue_gemm(zlm_device* d, zlm_resident* r, uint32_t quant, size_t rows, s
     float* ds = with_min ? reinterpret_cast<float*>(d->q_scratch + qbytes + fbytes) : nullptr;
     uint32_t rows32 = static_cast<uint32_t>(rows), m32 = static_cast<uint32_t>(m), nb32 = static_cast<uint32_t>(nb),
              mt32 = static_cast<uint32_t>(mt);
+    if (wide) {
+        const uint8_t* wq = r->gemm_payload;
+        const void* ws = r->gemm_scales;
+        void* qargs[] = {const_cast<float**>(&x_dev), &qx, &m32, &nb32};
+        // 256 slots a record, eight threads each
+        if (!launch(d, d->quantize_fp6, static_cast<unsigned>(records * 8), 256, qargs, "quantize tiled")) return false;
+        void* args[] = {&wq, &ws, &qx, &out_dev, &rows32, &m32, &nb32};
+        return launch3(d, d->gemm_wide, static_cast<unsigned>((rows + 191) / 192), static_cast<unsigned>(gt), 1, 768, args,
+                       "gemm wide");
+    }
     {
         const uint64_t n = mt * 32 * nb * 8;  // eight threads per (token, block)
         void* args[] = {const_cast<float**>(&x_dev), &qx, &dx, &m32, &nb32, &mt32, &ds};
@@ -1515,9 +1557,7 @@ bool enqueue_gemm(zlm_device* d, zlm_resident* r, uint32_t quant, size_t rows, s
     }
     const uint8_t* wq = r->gemm_payload;
     const void* ws = r->gemm_scales;
-    int split = 1;
-    const double tiled_us = gemm_tiled_us(qi, rows, m, nb, d->cus, &split);
-    if (m <= kGemmSmallM || gemm_small_us(qi, rows, m, nb, d->cus) < tiled_us) {
+    if (small) {
         // the split-K kernel, a workgroup per 32-row tile and 32-token tile
         const float* dsa = ds ? ds : dx;
         void* args[] = {&wq, &ws, &qx, &dx, &dsa, &out_dev, &rows32, &m32, &nb32};

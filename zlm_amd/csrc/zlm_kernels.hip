@@ -801,6 +801,81 @@ extern "C" __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_pe
 }
 
 
+#include "gemm_fp6.h"
+
+// ---- the wide fp6 GEMM -------------------------------------------------------
+
+// Its activations (gemm_fp6.h): the tiled quantizer's arithmetic into a record per
+// 128 tokens and block pair: the blocks' q as fp6 hi and lo parts, dx, dx * sum q.
+// Bound by the reads of x (17 us at 1999 tokens x 4096).  The codes' fields interleave four threads' elements (fp6_expand's order: field 4q + c
+// from the thread of place c, its elements permuted), so the threads transpose
+// their codes in two exchanges, each then holding 24 bits of four fields, and
+// three of each four store a dword of the hi and one of the lo codes.
+extern "C" __global__ void __launch_bounds__(256)
+    zlm_quantize_fp6_tiled(const float* __restrict__ x, uint8_t* __restrict__ qx, uint32_t m, uint32_t nb) {
+    // slots (32 tokens x 2 blocks x 4 tiles per record), eight threads each; the
+    // grid covers whole records
+    const uint64_t i = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+    const uint64_t slot = i / 8, record = slot / 256;
+    const uint32_t part = static_cast<uint32_t>(i % 8), npair = (nb + 1) / 2;
+    const uint32_t lt = static_cast<uint32_t>(slot % 32), blk = static_cast<uint32_t>(slot / 32 % 2),
+                   tile = static_cast<uint32_t>(slot / 64 % 4);
+    const uint32_t b = static_cast<uint32_t>(record % npair) * 2 + blk;
+    const uint64_t t = record / npair * 128 + tile * 32 + lt;
+    float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    if (t < m && b < nb) v = reinterpret_cast<const float4*>(x + (t * nb + b) * 32)[part];
+    float d;
+    int32_t s;
+    const uint32_t wv = q8_quant4(v, d, s);
+    s = sum8(s);
+    uint32_t hi = 0, lo = 0;  // four codes, a byte each
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const int q = static_cast<int8_t>(wv >> (8 * j));
+        const int h = (q + 8) >> 4;
+        hi |= fp6_code(h) << (8 * j);
+        lo |= fp6_code(q - 16 * h) << (8 * j);
+    }
+    // parts 0, 5, 4, 1 are places 0-3 of the record's first 16 fields, 2, 7, 6, 3 of the second
+    const uint32_t b0 = part & 1, b2 = part >> 2, second = (part >> 1) & 1;
+    const uint32_t place = b2 ? (b0 ? 1u : 2u) : (b0 ? 3u : 0u), place1 = b2 ? (b0 ? 2u : 1u) : (b0 ? 0u : 3u);  // part ^ 1's
+    const uint32_t order = place == 2 ? 0x02030001u : place == 3 ? 0x03000102u : 0x01020300u;
+    hi = __builtin_amdgcn_perm(0, hi, order);  // byte q: the code of field 4q + place
+    lo = __builtin_amdgcn_perm(0, lo, order);
+    const uint32_t even = __builtin_amdgcn_perm(lo, hi, 0x06040200u), odd = __builtin_amdgcn_perm(lo, hi, 0x07050301u);
+    const uint32_t keep = b0 ? odd : even;
+    const uint32_t got = __shfl_xor(b0 ? even : odd, 1, kWave);
+    auto pair = [&](int k) { return (((keep >> (8 * k)) & 63u) << (6 * place)) | (((got >> (8 * k)) & 63u) << (6 * place1)); };
+    const uint32_t h0 = pair(0), h1 = pair(1), l0 = pair(2), l1 = pair(3);  // quarters b0 and b0 + 2
+    hi = (b2 ? h1 : h0) | __shfl_xor(b2 ? h0 : h1, 4, kWave);
+    lo = (b2 ? l1 : l0) | __shfl_xor(b2 ? l0 : l1, 4, kWave);
+    const uint32_t q = b0 + 2 * b2, q1 = (q + 1) & 3;  // this thread's quarter (24 bits) and the next one's thread
+    const int next = static_cast<int>((threadIdx.x & 56u) | (q1 & 1u) | (second << 1) | ((q1 >> 1) << 2));
+    const uint32_t hn = __shfl(hi, next, kWave), ln = __shfl(lo, next, kWave);
+    uint8_t* o = qx + record * kFp6Record;
+    if (q < 3) {
+        const uint32_t w = 3 * second + q;  // dword of the 24 bytes: 0-3 in the first run, 4-5 in the second
+        const uint32_t at = w < 4 ? (tile * 2 + blk) * 1024 + w * 4 : kFp6Tail + (tile * 2 + blk) * 512 + (w - 4) * 4;
+        const uint32_t bytes = w < 4 ? 16 : 8, swap = w < 4 ? 0 : 32 * blk;  // the second block's tails: halves exchanged
+        *reinterpret_cast<uint32_t*>(o + at + (lt ^ swap) * bytes) = (hi >> (8 * q)) | (hn << (24 - 8 * q));
+        *reinterpret_cast<uint32_t*>(o + at + ((lt + 32) ^ swap) * bytes) = (lo >> (8 * q)) | (ln << (24 - 8 * q));
+    }
+    if (part == 0) {
+        float* dx = reinterpret_cast<float*>(o + kFp6Dx) + (tile * 2 + blk) * 32 + lt;
+        *dx = d;
+        dx[(kFp6Xs - kFp6Dx) / 4] = d * static_cast<float>(s);
+    }
+}
+
+// q4_1 and q4_k alike: their tiles hold the same nibbles and f32 (scale, min) pairs.
+// (The occupancy is stated twice: without the second the sums spill.)
+extern "C" __global__ void __launch_bounds__(kFp6Waves * 64)
+__attribute__((amdgpu_waves_per_eu(3, 3)))
+    zlm_gemm_wide(const uint8_t* __restrict__ wq, const uint8_t* __restrict__ ws, const uint8_t* __restrict__ qx,
+                  float* __restrict__ out, uint32_t rows, uint32_t m, uint32_t nb) {
+    gemm_fp6(wq, ws, qx, out, rows, m, nb);
+}
+
 // ---- small-M prefill GEMM (verify and microbatch batches, short prompts) -----
 // The same int path and tiled operands as gemm_tiles, one 32-token tile per
 // workgroup (grid.y: the token tiles).
