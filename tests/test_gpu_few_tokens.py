@@ -24,7 +24,7 @@ matvec/layout.zig:458-476): the int-path token GEMV (zlm_gemv_<quant>_q8tok4_
 g<T>, two-row tiles for the nibble quants from 32768 rows) quantizes the
 activations in its own prologue; m = 5..8 its eight-slot form for q4_1 at k
 <= 4096 and q4_k there up to 8192 rows, the small-M GEMM otherwise (both
-checked here at m = 5 and 8).  Against the oracle's int
+checked here at m = 5 and 8), tall nibble weights the tall kernel.  Against the oracle's int
 path (orc_matmul_int) at relative L2 <= 1e-5, which one activation off by one
 quantization unit would exceed, with activations that stress the quantizer
 (a zero block, a block with one nonzero, values near rounding ties and a
@@ -157,6 +157,47 @@ def test_int_tokens_match_oracle(dev, qt, zq, rows, k, m):
         mag = np.abs(x.reshape(m, k).astype(np.float64)) @ dq.T
         assert np.all(np.abs(out.reshape(m, rows) - fp) <= 0.02 * mag + 1e-6)
     finally:
+        dev.free_resident(res)
+
+
+# The tall kernel (16-row tiles of the GEMV layout): a last tile of 1, 15 and 16
+# rows, its x tiers' ends (4096 | 4352, 8192), iterations that end inside a row
+# (k = 64, 320: q4_0 / q4_1 only), one token set and two, the last row of x.
+TALL_CASES = [(synth.Q4_K, 65536 + 1, 256, 3), (synth.Q4_K, 32768, 4096, 5), (synth.Q4_K, 32768 + 15, 4352, 8),
+              (synth.Q4_K, 65536 + 1, 8192, 4), (synth.Q4_0, 65536 + 1, 64, 4), (synth.Q4_0, 65536 + 15, 320, 5),
+              (synth.Q4_0, 65536, 4096, 8), (synth.Q4_0, 65536 + 1, 4160, 6), (synth.Q4_1, 65536 + 15, 2048, 3),
+              (synth.Q4_1, 32768 + 1, 320, 7), (synth.Q4_1, 32768, 8192, 8)]
+
+
+@pytest.mark.parametrize("qt,rows,k,m", TALL_CASES)
+def test_tall_tokens(dev, qt, rows, k, m):
+    zq = dict(QUANTS)[qt]
+    _say(f"tall tokens type={qt} rows={rows} k={k} m={m}")
+    w = synth.weights(qt, rows, k, seed=rows + k + m)
+    xs = _stress_x(m, k, rows + m) if k >= 128 else synth.activation(m, m * k)
+    res = dev.upload_resident(w)
+    x = dev.dev_malloc(xs.nbytes)
+    out = dev.dev_malloc(m * rows * 4)
+    try:
+        dev.dev_upload(x, xs)
+        dev.dev_upload(out, np.full(m * rows, np.nan, np.float32))
+        assert dev.launch_log(True)
+        assert dev.mat_mul_enqueue(res, zd.quant(zq), rows, k, m, x, out), dev.last_error()
+        dev.sync()
+        assert [r["what"] for r in dev.launch_log_read() if "repack" not in r["what"]][-1] == "gemm tall"
+        got = np.zeros(m * rows, np.float32)
+        dev.dev_download(got, out)
+        got = got.reshape(m, rows)
+        assert np.all(np.isfinite(got))
+        rb = synth.row_bytes(qt, k)
+        # f32 sums of at most 256 block terms per output: a few of their roundings
+        for r0, r1 in ((0, 32), (rows // 2, rows // 2 + 48), (rows - 512, rows)):
+            want = oracle.matmul_int(qt, w[r0 * rb:r1 * rb], k, r1 - r0, m, xs)
+            assert rel_l2(got[:, r0:r1], want) <= 2e-6, (r0, r1)
+    finally:
+        dev.launch_log(False)
+        dev.dev_free(x)
+        dev.dev_free(out)
         dev.free_resident(res)
 
 

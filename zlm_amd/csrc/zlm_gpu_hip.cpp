@@ -204,6 +204,8 @@ struct zlm_device {
     // the wide fp6 GEMM (q4_1 / q4_k; 128-token x 192-row tiles, 12 waves) and its activations
     hipFunction_t quantize_fp6 = nullptr;
     hipFunction_t gemm_wide = nullptr;
+    // 3 to 8 tokens by a tall weight, from the GEMV layout: k up to 4096, up to 8192
+    hipFunction_t gemm_tall[kNumQuants][2] = {};
     hipFunction_t qk_norm_rope_kv = nullptr;
     hipFunction_t attn_partial = nullptr;
     hipFunction_t attn_combine = nullptr;
@@ -306,6 +308,9 @@ void unload_modules(zlm_device* d) {
     d->gemv.clear();
 }
 
+// The quants the tall kernel has (below, enqueue_gemm_tall).
+bool gemm_tall_type(uint32_t type) { return type == ZLM_GGML_Q4_0 || type == ZLM_GGML_Q4_1 || type == ZLM_GGML_Q4_K; }
+
 bool load_kernels(zlm_device* d) {
     const std::string dir = library_dir();
     const char* env = getenv("ZLM_HIP_CODE_OBJECT");
@@ -359,6 +364,14 @@ bool load_kernels(zlm_device* d) {
                 {&d->synth_f16, "zlm_synth_f16"}};
     for (const auto& m : more)
         if (!ok(d, hipModuleGetFunction(m.f, d->mod, m.name), m.name)) return false;
+    for (const QuantInfo& qi : kQuants) {
+        if (!gemm_tall_type(qi.type)) continue;
+        for (int tier = 0; tier < 2; tier++) {
+            char nm[64];
+            snprintf(nm, sizeof nm, "zlm_gemm_tall_%s_g%d", kQuantNames[qi.slot], tier ? 8 : 4);
+            if (!ok(d, hipModuleGetFunction(&d->gemm_tall[qi.slot][tier], d->mod, nm), nm)) return false;
+        }
+    }
     return true;
 }
 
@@ -1490,6 +1503,34 @@ bool ensure_gemm_tiles(zlm_device* d, zlm_resident* r, const QuantInfo* qi, uint
 // Q4_1 or Q4_K weight and device activations x_dev (m x k, token-major):
 // quantize x to q8 blocks into the tiled device scratch (plus dx*sum(q) for
 // the min-carrying types), then the int8-MFMA GEMM over the tiled weights.
+// The tall kernel (16-row tiles of the GEMV layout, a wave each, one 16-wave
+// workgroup per CU; no tiled copy, no quantizer launch) runs m = 3..8 where there
+// are tiles enough for the chip's 4096 waves: a tile is one wave's, so a call takes
+// at least as long as a tile, 1.6 us per 256 elements.  Measured, before and with
+// it, us: q4_k m = 8 32768 x 4096 35 and 28, x 1024 15 and 11, 24576 x 3840 26 and
+// 28; q4_1 m = 8 32768 x 4096 36 and 32, 24576 x 3840 30 and 27, 16384 x 4096 23 and
+// 32; q4_0 m = 8 65536 x 4096 42 and 32, 49152 x 4096 33 and 32, 32768 x 4096 23 and
+// 31.  At m = 3 and 4 the int token GEMV is closer: q4_k 65536 x 4096 42 and 32,
+// 65536 x 8192 80 and 75, 32768 x 4096 25 and 28; q4_0 and q4_1 win only with short
+// rows (q4_0 262144 x 2048 69 and 64, 65536 x 2048 22 and 19; 151936 x 4096 73 and 76,
+// 65536 x 8192 63 and 68).  k % 64: q4_0 and q4_1 scales are loaded in pairs.
+bool gemm_tall_pays(const QuantInfo* qi, size_t rows, size_t k, size_t m) {
+    if (!gemm_tall_type(qi->type) || m < 3 || m > 8 || k > 8192 || k % 64) return false;
+    if (m <= 4) return rows >= 65536 && (qi->type == ZLM_GGML_Q4_K || k <= 2048);
+    return rows >= (qi->type == ZLM_GGML_Q4_0 ? 65536 : 32768);
+}
+
+bool enqueue_gemm_tall(zlm_device* d, zlm_resident* r, const QuantInfo* qi, size_t rows, size_t k, size_t m,
+                       const float* x_dev, float* out_dev) {
+    const uint8_t* w = r->payload;
+    const uint16_t* s = r->scales;
+    uint32_t rows32 = static_cast<uint32_t>(rows), m32 = static_cast<uint32_t>(m), nb32 = static_cast<uint32_t>(k / 32);
+    void* args[] = {&w, &s, const_cast<float**>(&x_dev), &out_dev, &rows32, &m32, &nb32};
+    const uint64_t wgs = (static_cast<uint64_t>(rows) + 255) / 256;  // 16 tiles of 16 rows each
+    const unsigned grid = static_cast<unsigned>(std::min<uint64_t>(wgs, static_cast<uint64_t>(d->cus)));
+    return launch(d, d->gemm_tall[qi->slot][k <= 4096 ? 0 : 1], grid, 1024, args, "gemm tall");
+}
+
 bool enqueue_gemm(zlm_device* d, zlm_resident* r, uint32_t quant, size_t rows, size_t k, size_t m,
                   const float* x_dev, float* out_dev) {
     if (!d || !d->avail) return fail(d, "device unavailable");
@@ -1513,6 +1554,7 @@ bool enqueue_gemm(zlm_device* d, zlm_resident* r, uint32_t quant, size_t rows, s
             if (!enqueue_gemv(d, r, quant, rows, k, x_dev + t * k, out_dev + t * rows)) return false;
         return true;
     }
+    if (gemm_tall_pays(qi, rows, k, m)) return enqueue_gemm_tall(d, r, qi, rows, k, m, x_dev, out_dev);
     {  // a few tokens: the int path in one pass over the GEMV layout, no tiled copy or quantizer launch
         bool ran = false;
         if (!enqueue_gemv_q8tok(d, r, qi, rows, k, m, x_dev, out_dev, &ran)) return false;

@@ -1038,6 +1038,22 @@ ZLM_GEMM_SMALL(zlm_gemm_small_q8_0_q8, Q8_0, uint16_t)
 ZLM_GEMM_SMALL(zlm_gemm_small_q4_1_q8, Q4_1, float2)
 ZLM_GEMM_SMALL(zlm_gemm_small_q4_k_q8, Q4_K, float2)
 
+// ---- a few tokens by a tall weight -------------------------------------------
+#include "gemm_tall.h"
+
+#define ZLM_GEMM_TALL(NAME, QT, KCAP)                                                                          \
+    extern "C" __global__ void __launch_bounds__(kTallWaves * 64)                                        \
+        NAME(const uint8_t* __restrict__ w, const uint8_t* __restrict__ d, const float* __restrict__ x,        \
+             float* __restrict__ out, uint32_t rows, uint32_t m, uint32_t nb) {                                \
+        gemm_tall<QT, KCAP>(w, d, x, out, rows, m, nb);                                                        \
+    }
+ZLM_GEMM_TALL(zlm_gemm_tall_q4_0_g4, Q4_0, 4096)
+ZLM_GEMM_TALL(zlm_gemm_tall_q4_1_g4, Q4_1, 4096)
+ZLM_GEMM_TALL(zlm_gemm_tall_q4_k_g4, Q4_K, 4096)
+ZLM_GEMM_TALL(zlm_gemm_tall_q4_0_g8, Q4_0, 8192)
+ZLM_GEMM_TALL(zlm_gemm_tall_q4_1_g8, Q4_1, 8192)
+ZLM_GEMM_TALL(zlm_gemm_tall_q4_k_g8, Q4_K, 8192)
+
 // ---- decode-step glue -------------------------------------------------------
 // The non-GEMV ops of one Qwen3 decode layer (reference
 // architectures/impl/qwen3/block.zig:20-41), so activations stay in HBM
