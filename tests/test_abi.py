@@ -151,6 +151,24 @@ def test_profiler_check_reads_the_process_map(tmp_path):
     assert not zd.profiler_loaded()
 
 
+def test_profiler_check_sees_later_loads(tmp_path):
+    """The process's own map is read again only when the loader's object counts
+    change: a library of a profiler's name (an empty one, in a process of its
+    own) is seen when it is loaded after a check, and gone after it is closed."""
+    import subprocess
+    import sys
+    src = tmp_path / "empty.c"
+    src.write_text("int zlm_empty;\n")
+    fake = tmp_path / "librocprofiler-sdk-empty.so"
+    subprocess.run(["gcc", "-shared", "-fPIC", str(src), "-o", str(fake)], check=True)
+    code = ("import _ctypes\nfrom zlm_amd import device as zd\n"
+            "assert not zd.profiler_loaded() and not zd.profiler_loaded()\n"
+            f"h = _ctypes.dlopen({str(fake)!r}, 0)\n"
+            "assert zd.profiler_loaded() and zd.profiler_loaded()\n"
+            "_ctypes.dlclose(h)\nassert not zd.profiler_loaded()\n")
+    subprocess.run([sys.executable, "-c", code], check=True, cwd=os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
+
+
 def _kernel_args(path):
     """{kernel name: [sizes of its explicit arguments]} from a code object's
     metadata (the ROCm LLVM tools read the bundle and the ELF notes)."""
