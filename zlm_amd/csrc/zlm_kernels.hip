@@ -1194,13 +1194,17 @@ constexpr int kAttnSplit = 64;
 constexpr int kAttnPart = kAttnHd + 2;
 
 // V tile row stride in dwords: 64 positions + 4, so the 16 lanes of one
-// 128-bit LDS read pass (columns l..l+15, same positions) cover all 64 banks.
+// 128-bit LDS read pass (columns l..l+15, same positions) cover all 64 banks;
+// 16 more past every 16 columns, so that the staging lanes (16 positions of each
+// column group) cover them too (a group's 16 * 68 dwords alone are whole rounds of
+// the banks: four lanes a bank).
 constexpr int kAttnVStride = kAttnSplit + 4;
+__device__ __forceinline__ uint32_t attn_v_at(uint32_t column) { return column * kAttnVStride + column / 16 * 16; }
 
 struct alignas(16) AttnLds {
     float qs[4][kAttnHd];                          // scaled q of the G heads (zeros past G)
     float sc[4][kAttnSplit];                       // scores
-    uint32_t vt[kAttnHd / 2][kAttnVStride];        // V transposed: [dim pair][position] f16 pairs
+    uint32_t vt[kAttnHd / 2 * kAttnVStride + 48];  // V transposed: f16 pairs, dim pair c at attn_v_at(c) + position
 };
 
 // Position-independent K and V loads of thread (p, qd) of split t0.
@@ -1226,7 +1230,7 @@ __device__ __forceinline__ void attn_stage_v(const uint4 (&vraw)[4], uint32_t p,
     for (int c = 0; c < 4; c++) {
         const uint32_t w[4] = {vraw[c].x, vraw[c].y, vraw[c].z, vraw[c].w};
 #pragma unroll
-        for (int i = 0; i < 4; i++) sm.vt[16 * qd + 4 * c + i][p] = valid ? w[i] : 0u;
+        for (int i = 0; i < 4; i++) sm.vt[attn_v_at(16 * qd) + (4 * c + i) * kAttnVStride + p] = valid ? w[i] : 0u;
     }
 }
 
@@ -1294,7 +1298,7 @@ __device__ __forceinline__ void attn_values(const AttnLds& sm, uint32_t g, uint3
     float a0 = 0.0f, a1 = 0.0f;
 #pragma unroll
     for (int j4 = 0; j4 < kAttnSplit; j4 += 4) {
-        const uint4 v = *reinterpret_cast<const uint4*>(&sm.vt[lane][j4]);
+        const uint4 v = *reinterpret_cast<const uint4*>(&sm.vt[attn_v_at(lane) + j4]);
         const uint32_t vw[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
         for (int i = 0; i < 4; i++) {
@@ -1339,9 +1343,9 @@ extern "C" __global__ void __launch_bounds__(256)
         const uint32_t i = tid + 256u * j, g = i / kAttnHd;
         sm.qs[g][i % kAttnHd] = g < G ? qv[j] * scale : 0.0f;
     }
-    attn_stage_v(vraw, p, qd, valid, kAttnSplit, sm);
-    __syncthreads();
+    sk_barrier();
     attn_scores<false>(kraw, p, qd, valid, kAttnSplit, nullptr, sm);
+    attn_stage_v(vraw, p, qd, valid, kAttnSplit, sm);
     __syncthreads();
     if (wid < G) attn_values(sm, wid, lane, part + (static_cast<size_t>(h * G + wid) * nsplit + s) * kAttnPart);
 }
@@ -1481,6 +1485,11 @@ extern "C" __global__ void __launch_bounds__(1024)
 //     loaded slice in the scores);
 //   * scores, softmax and values as zlm_attn_partial, into the same partials,
 //     which zlm_attn_combine merges.
+// Bound by one memory round trip and the chain behind it, so the rotary angles and
+// the q heads are done while the K and V slices are on their way (their barriers
+// wait for LDS only), and V is staged last, behind the scores.  Staged first, and
+// with four lanes a bank: 12.6 us with its merge at 8000 positions of 32 heads over
+// 8, now 12.3; in a 36-layer step at 2048 positions 1759 us, now 1714.
 // nsplit may cover fewer positions than the cache holds (a window: the host
 // launches ceil(window / 64) splits for steps whose position is below it).  A
 // position past the launched splits would leave positions out, so the first
@@ -1529,17 +1538,7 @@ extern "C" __global__ void __launch_bounds__(256)
         cs[tid] = cosf(angle);
         sn[tid] = sinf(angle);
     }
-    attn_stage_v(vraw, p, qd, valid, prow, sm);
-    if (own && wid == 1) {  // the new V row, as the f16 values the cache holds
-        const _Float16 e0 = static_cast<_Float16>(v0), e1 = static_cast<_Float16>(v1);
-        _Float16* vd = vc + (static_cast<size_t>(h) * max_seq + pos_i) * kAttnHd;
-        vd[lane] = e0;
-        vd[lane + half] = e1;
-        // dim d sits in half d%2 of dword column d/2 at position prow
-        reinterpret_cast<_Float16*>(&sm.vt[lane / 2][prow])[lane % 2] = e0;
-        reinterpret_cast<_Float16*>(&sm.vt[(lane + half) / 2][prow])[lane % 2] = e1;
-    }
-    __syncthreads();
+    sk_barrier();
     // q head g: RMSNorm, rotate, scale (lane l owns the pair (l, l + 64))
     if (wid < G) {
         const float inv = 1.0f / sqrtf(wave_sum(fmaf(q0, q0, q1 * q1)) / static_cast<float>(kAttnHd) + eps);
@@ -1562,8 +1561,18 @@ extern "C" __global__ void __launch_bounds__(256)
         kn[lane] = static_cast<float>(r0);
         kn[lane + half] = static_cast<float>(r1);
     }
-    __syncthreads();
+    sk_barrier();
     attn_scores<true>(kraw, p, qd, valid, prow, kn, sm);
+    attn_stage_v(vraw, p, qd, valid, prow, sm);
+    if (own && wid == 1) {  // the new V row, as the f16 values the cache holds
+        const _Float16 e0 = static_cast<_Float16>(v0), e1 = static_cast<_Float16>(v1);
+        _Float16* vd = vc + (static_cast<size_t>(h) * max_seq + pos_i) * kAttnHd;
+        vd[lane] = e0;
+        vd[lane + half] = e1;
+        // dim d sits in half d%2 of dword column d/2 at position prow
+        reinterpret_cast<_Float16*>(&sm.vt[attn_v_at(lane / 2) + prow])[lane % 2] = e0;
+        reinterpret_cast<_Float16*>(&sm.vt[attn_v_at((lane + half) / 2) + prow])[lane % 2] = e1;
+    }
     __syncthreads();
     const bool past_window = L > nsplit * kAttnSplit;
     if (wid < G)
