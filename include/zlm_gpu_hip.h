@@ -221,7 +221,8 @@ bool zlm_gpu_vram_info(zlm_device *dev, uint64_t *free_bytes, uint64_t *total_by
  * then the device layout, plus the prefill GEMM's tiled copy once the tiled
  * GEMM has run on it (more than 4 tokens, or 3-4 tokens at k > 8192, k >
  * 16384 for Q4_1 / Q4_K; fewer tokens, and 5-8 tokens where the eight-slot
- * int-path GEMV runs, read the device layout). */
+ * int-path GEMV runs and 3-8 tokens by a tall q4_0, q4_1 or q4_k weight (the
+ * tall kernel: from 32768 rows up, k <= 8192), read the device layout). */
 uint64_t zlm_gpu_resident_device_bytes(const zlm_resident *res);
 /* HBM a rows x k weight of `quant` will hold once converted (its device
  * layout), plus its GEMM tiled copy when `with_gemm` (tensors the plan also
@@ -411,7 +412,9 @@ bool zlm_gpu_attention_decode_enqueue_noalloc(zlm_device *dev, const float *qkv,
  * timers) fail while a capture is open.  Ops that allocate or convert layouts
  * on first use (a resident's first op, a resident's first matMul, the
  * attention and GEMM scratch) must have run once eagerly before their
- * capture; under capture they fail instead.  The library never frees or
+ * capture; under capture they fail instead (a matMul of up to 8 tokens may
+ * need neither tiles nor scratch and then builds none, so a wider one must
+ * have run eagerly itself).  The library never frees or
  * replaces scratch that a captured graph references while that graph exists:
  * after capturing an attention call, an eager attention call that needs more
  * partials fails with the reason; after capturing a matMul, an eager matMul

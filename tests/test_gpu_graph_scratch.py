@@ -10,7 +10,8 @@ fresh device (so these calls size the scratch themselves):
   destroyed the larger call runs and matches the oracle;
 * matMul (the prefill GEMM): the same with the activation scratch and a
   resident's GEMM tiles, replays checked against the eager result and the
-  oracle's int path (oracle.matmul_int);
+  oracle's int path (oracle.matmul_int); a product whose wide form needs more
+  scratch than its tiled form runs the tiled one where the scratch cannot grow;
 * the host-buffer contract ops refuse to run under capture.
 """
 import math
@@ -176,6 +177,67 @@ def test_gemm_scratch_outlives_its_graph(fresh):
             dev.graph_destroy(graph)
         for p in (d_xs, d_xb, d_os, d_ob):
             dev.dev_free(p)
+        dev.free_resident(res)
+
+
+def test_wide_gemm_falls_back_where_its_scratch_cannot_grow(fresh):
+    """The wide fp6 GEMM's activations take 1.4 times the tiled form's scratch."""
+    dev = fresh
+    rows, k, m = 56 * 192, 1536, 512
+    q = zd.quant(zd.Q4_1)
+    w = synth.weights(synth.Q4_1, rows, k, seed=57)
+    x = synth.activation(58, m * k)
+    res = dev.upload_resident(w)
+    assert res is not None, dev.last_error()
+    d_x, d_o = dev.dev_malloc(x.nbytes), dev.dev_malloc(m * rows * 4)
+    dev.dev_upload(d_x, x)
+    want = oracle.matmul_int(synth.Q4_1, w[:32 * synth.row_bytes(synth.Q4_1, k)], k, 32, m, x)
+    graph = None
+
+    def check():
+        got = np.zeros(m * rows, np.float32)
+        dev.dev_download(got, d_o)
+        assert rel_l2(got.reshape(m, rows)[:, :32], want) <= 1e-6  # f32 sums of 48 block terms
+
+    def whats():
+        return [r["what"] for r in dev.launch_log_read() if r["what"].startswith("gemm")]
+
+    try:
+        _say("graph scratch: a product of few rows builds the tiles and the tiled form's scratch")
+        assert dev.mat_mul_enqueue(res, q, 640, k, m, d_x, d_o), dev.last_error()
+        sized = dev.scratch_device_bytes()
+        assert dev.launch_log(True)
+        assert dev.capture_begin(), dev.last_error()
+        try:
+            ok = dev.mat_mul_enqueue(res, q, rows, k, m, d_x, d_o)
+        finally:
+            graph = dev.capture_end()
+        assert ok and graph is not None, dev.last_error()
+        assert "gemm wide" not in whats()
+        for _ in range(3):
+            dev.dev_upload(d_o, np.zeros(m * rows, np.float32))
+            dev.graph_launch(graph, 1)
+            check()
+        _say("graph scratch: beside the graph, eagerly")
+        assert dev.launch_log(True)
+        assert dev.mat_mul_enqueue(res, q, rows, k, m, d_x, d_o), dev.last_error()
+        assert "gemm wide" not in whats()
+        check()
+        assert dev.scratch_device_bytes() == sized
+        dev.graph_destroy(graph)
+        graph = None
+        _say("graph scratch: after the graph is destroyed the scratch grows")
+        assert dev.launch_log(True)
+        assert dev.mat_mul_enqueue(res, q, rows, k, m, d_x, d_o), dev.last_error()
+        assert whats() == ["gemm wide"]
+        check()
+        assert dev.scratch_device_bytes() > sized
+    finally:
+        dev.launch_log(False)
+        if graph is not None:
+            dev.graph_destroy(graph)
+        dev.dev_free(d_x)
+        dev.dev_free(d_o)
         dev.free_resident(res)
 
 

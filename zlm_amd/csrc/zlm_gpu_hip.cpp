@@ -1569,13 +1569,20 @@ bool enqueue_gemm(zlm_device* d, zlm_resident* r, uint32_t quant, size_t rows, s
     int split = 1;
     const double tiled_us = gemm_tiled_us(qi, rows, m, nb, d->cus, &split);
     const bool small = m <= kGemmSmallM || gemm_small_us(qi, rows, m, nb, d->cus) < tiled_us;
-    const bool wide = !small && gemm_wide_pays(qi, rows, m, nb, d->cus, tiled_us);
     const uint64_t mt = (static_cast<uint64_t>(m) + 31) / 32;
-    // the wide kernel's activations: records of 128 tokens and two blocks
-    const uint64_t gt = (static_cast<uint64_t>(m) + 127) / 128, records = gt * ((nb + 1) / 2);
     const uint64_t qbytes = mt * 32 * k;  // a multiple of 1024
     const uint64_t fbytes = mt * 32 * nb * 4;
-    const uint64_t need = wide ? records * 14336 : qbytes + fbytes * (with_min ? 2 : 1);
+    const uint64_t need = qbytes + fbytes * (with_min ? 2 : 1);
+    // The wide kernel's activations: records of 128 tokens and two blocks, 1.4 times
+    // the tiled form's bytes.  Where the scratch holds the tiled form but cannot grow
+    // for the records (under capture, beside a graph that uses it, memory spent), or a
+    // launch could not cover them, the tiled kernels run.
+    const uint64_t gt = (static_cast<uint64_t>(m) + 127) / 128, records = gt * ((nb + 1) / 2);
+    bool wide = !small && records < (1u << 21) && gemm_wide_pays(qi, rows, m, nb, d->cus, tiled_us);
+    if (wide && records * 14336 > d->q_scratch_cap) {
+        wide = !d->capturing && d->gemm_graphs == 0 && ensure_bytes(d, d->q_scratch, d->q_scratch_cap, records * 14336);
+        if (!wide) hipGetLastError();
+    }
     if (need > d->q_scratch_cap && !may_replace_scratch(d, kUsesGemm, "the GEMM activation scratch")) return false;
     if (!ensure_bytes(d, d->q_scratch, d->q_scratch_cap, need)) return false;
     if (d->capturing) d->capture_uses |= kUsesGemm;
