@@ -351,3 +351,33 @@ def test_resident_device_bytes_follow_the_conversions(dev):
         assert dev.mat_mul_resident(res, zd.quant(zq), rows, k, m, x, again), dev.last_error()
         np.testing.assert_array_equal(again, outm)
         dev.free_resident(res)
+
+
+# A host matMul's x comes by the copy kernel up to 896 KiB and by DMA past it, its
+# y is stored into host memory up to 12 MiB (1 MiB for one and two tokens), then
+# copied by DMA: either side of each line, odd rows among them.
+@pytest.mark.parametrize("rows,k,m,staged", [(63, 64, 1, True), (131071, 64, 2, True), (131073, 64, 2, True),
+                                             (65, 4096, 56, True), (65, 4096, 57, False), (40001, 32, 78, True),
+                                             (40001, 32, 79, True), (63, 7168, 32, True), (63, 7200, 32, False)])
+def test_host_matmul_copies(dev, rows, k, m, staged):
+    _say(f"host matmul copies rows={rows} k={k} m={m}")
+    w = synth.weights(synth.Q4_0, rows, k, seed=rows + m)
+    x = synth.activation(k + m, m * k)
+    res = dev.upload_resident(w)
+    x_dev, out_dev = dev.dev_malloc(x.nbytes), dev.dev_malloc(m * rows * 4)
+    try:
+        dev.dev_upload(x_dev, x)
+        want = np.zeros(m * rows, np.float32)
+        assert dev.mat_mul_enqueue(res, zd.quant(zd.Q4_0), rows, k, m, x_dev, out_dev), dev.last_error()
+        dev.dev_download(want, out_dev)
+        assert dev.launch_log(True)
+        for _ in range(2):  # the second on buffers that hold the first's
+            out = np.full(m * rows, np.nan, np.float32)
+            assert dev.mat_mul_resident(res, zd.quant(zd.Q4_0), rows, k, m, x, out), dev.last_error()
+            np.testing.assert_array_equal(out.view(np.uint32), want.view(np.uint32))
+        assert ("stage x" in [r["what"] for r in dev.launch_log_read()]) == staged
+    finally:
+        dev.launch_log(False)
+        dev.dev_free(x_dev)
+        dev.dev_free(out_dev)
+        dev.free_resident(res)

@@ -1997,21 +1997,41 @@ extern "C" bool zlm_gpu_mat_vec_resident_batch(zlm_device* d, size_t k, const fl
     return true;
 }
 
+// How a host matMul's x and y cross: small ones are bound by the DMA copies' own
+// start and end (6 and 9 us), not by their bytes, so the copy kernel pulls x and the
+// product stores y straight into pinned host memory, as in the GEMV ops; large ones
+// by the bytes, which the DMA engine moves better.  Measured, us of the whole call,
+// DMA both ways and direct:
+//   q4_0 4096 x 4096 x 4 39 and 26, 12288 x 4096 x 8 60 and 46, 12288 x 4096 x 2 44
+//   and 32; q4_k 12288 x 4096 x 24 124 and 105, 262144 x 3840 x 5 413 and 329.
+//   x by the copy kernel: 896 KiB 105 -> 104 (q8_0 4096 x 4096 x 56), 1 MiB 102 -> 104
+//   (q4_0 4096 x 16384 x 16), 3.1 MiB 655 -> 680 (12288 x 4096 x 200).
+//   y from the product: 9.4 MiB 660 -> 640 (q4_0 12288 x 4096 x 200), 11.4 MiB 800 ->
+//   735 (q8_0 20000 x 4096 x 150), 24 MiB 1620 -> 1643 (12288 x 4096 x 512).  From the
+//   one- and two-token GEMVs, whose waves store a few rows at a time: 0.5 MiB 96 -> 86
+//   (q4_k 65536 x 3840), 1.2 MiB 181 -> 187 (q4_0 151936 x 4096).
+constexpr size_t kMatMulStageBytes = 896u << 10, kMatMulDirectBytes = 12u << 20, kMatMulDirectGemvBytes = 1u << 20;
+
 extern "C" bool zlm_gpu_mat_mul_resident(zlm_device* d, zlm_resident* r, uint32_t quant, size_t rows, size_t k,
                                          size_t m, const float* x, size_t x_len, float* out, size_t out_len) {
     if (!contract_ready(d)) return false;
     if (!x || !out || m == 0 || x_len != m * k || out_len < m * rows) return fail(d, "bad buffers");
     if (!ensure_pair(d, d->d_x, d->h_x, d->x_cap, m * k, d->h_x_dev)) return false;
     if (!ensure_pair(d, d->d_y, d->h_y, d->y_cap, m * rows, d->h_y_dev)) return false;
-    memcpy(d->h_x, x, m * k * sizeof(float));
-    if (!ok(d, hipMemcpyAsync(d->d_x, d->h_x, m * k * sizeof(float), hipMemcpyHostToDevice, d->stream), "stage x"))
-        return false;
-    if (!enqueue_gemm(d, r, quant, rows, k, m, d->d_x, d->d_y)) {
+    if (m * k * sizeof(float) <= kMatMulStageBytes) {
+        if (!stage_x_sync(d, x, m * k)) return false;
+    } else {
+        memcpy(d->h_x, x, m * k * sizeof(float));
+        if (!ok(d, hipMemcpyAsync(d->d_x, d->h_x, m * k * sizeof(float), hipMemcpyHostToDevice, d->stream), "stage x"))
+            return false;
+    }
+    const bool direct = m * rows * sizeof(float) <= (m <= kGemmGemvM ? kMatMulDirectGemvBytes : kMatMulDirectBytes);
+    if (!enqueue_gemm(d, r, quant, rows, k, m, d->d_x, direct ? d->h_y_dev : d->d_y)) {
         hipStreamSynchronize(d->stream);
         return false;
     }
-    // the m x rows result (megabytes at prefill sizes) comes back by DMA
-    if (!ok(d, hipMemcpyAsync(d->h_y, d->d_y, m * rows * sizeof(float), hipMemcpyDeviceToHost, d->stream), "read y"))
+    if (!direct &&
+        !ok(d, hipMemcpyAsync(d->h_y, d->d_y, m * rows * sizeof(float), hipMemcpyDeviceToHost, d->stream), "read y"))
         return false;
     return finish_sync(d, out, m * rows);
 }
