@@ -1,0 +1,116 @@
+"""The host library's own decisions, without a GPU: zlm_gpu_hip.cpp built
+against a HIP runtime that allocates host memory under a limit and runs no
+kernels (tests/fake_hip.cpp).  What a call launches comes from the launch log,
+what it allocates, frees, copies and waits for from the runtime's counters.
+Numerical results of the same routes are the GPU tests' part."""
+import ctypes
+import importlib.util
+import os
+import subprocess
+import sys
+
+import numpy as np
+import pytest
+
+from zlm_amd import device as zd
+from zlm_amd import synth
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+LIVE, MALLOCS, REFUSED, FREES, SYNCS, H2D, D2H, MISUSE = range(8)
+NO_LIMIT = (1 << 64) - 1
+
+
+@pytest.fixture(scope="module")
+def fake(tmp_path_factory):
+    """The package's device module over the library built with the stand-in runtime."""
+    lib = tmp_path_factory.mktemp("fake_hip") / "libzlm_gpu_hip.so"
+    rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
+    subprocess.run(["g++", "-O1", "-std=c++17", "-fPIC", "-shared", "-w", "-D__HIP_PLATFORM_AMD__", f"-I{rocm}/include",
+                    f"-I{ROOT}/include", f"-I{ROOT}/zlm_amd/csrc", f"{ROOT}/zlm_amd/csrc/zlm_gpu_hip.cpp",
+                    f"{ROOT}/tests/fake_hip.cpp", "-Wl,-Bsymbolic", "-ldl", "-o", str(lib)], check=True)
+    spec = importlib.util.spec_from_file_location("zlm_device_fake_hip", zd.__file__)
+    mod = importlib.util.module_from_spec(spec)
+    sys.modules[spec.name] = mod
+    spec.loader.exec_module(mod)
+    mod.LIB_PATH = str(lib)
+    raw = mod.lib()
+    raw.fake_hip_stat.restype = ctypes.c_uint64
+    raw.fake_hip_limit.argtypes = [ctypes.c_uint64]
+    return mod
+
+
+class _Box:
+    """A device over the stand-in runtime, with device buffers for x and out."""
+
+    def __init__(self, mod, x_floats, out_floats):
+        self.raw = mod.lib()
+        self.raw.fake_hip_limit(NO_LIMIT)
+        self.dev = mod.Device()
+        assert self.dev.available(), self.dev.last_error()
+        self.misuse = self.stat(MISUSE)
+        self.x, self.out = self.dev.dev_malloc(4 * x_floats), self.dev.dev_malloc(4 * out_floats)
+
+    def stat(self, i):
+        return int(self.raw.fake_hip_stat(i))
+
+    def resident(self, qt, rows, k):
+        res = self.dev.upload_resident(np.zeros(rows * synth.row_bytes(qt, k), np.uint8))
+        assert res is not None
+        return res
+
+    def run(self, res, qt, rows, k, m):
+        """(accepted, the launches that do not convert weights)"""
+        assert self.dev.launch_log(True)
+        ok = self.dev.mat_mul_enqueue(res, zd.quant(qt), rows, k, m, self.x, self.out)
+        log = [r for r in self.dev.launch_log_read() if r["what"] not in ("repack", "repack records", "tile weights")]
+        return ok, log
+
+    def whats(self, *call):
+        ok, log = self.run(*call)
+        assert ok, self.dev.last_error()
+        return [r["what"] for r in log]
+
+
+@pytest.fixture
+def box(fake):
+    made = []
+
+    def make(x_floats, out_floats):
+        made.append(_Box(fake, x_floats, out_floats))
+        return made[-1]
+
+    yield make
+    for b in made:
+        assert b.stat(MISUSE) == b.misuse
+        b.raw.fake_hip_limit(NO_LIMIT)
+        b.dev.deinit()
+
+
+def test_wide_gemm_where_memory_is_spent(box):
+    """The wide GEMM's activations take more scratch than the tiled form's.  A
+    refused growth costs nothing that the call or a later one needs."""
+    qt, k, m = synth.Q4_1, 1536, 512
+    rows = 56 * 192
+    b = box(m * k, m * rows)
+    res = b.resident(qt, rows, k)
+    spare = b.dev.dev_malloc(1 << 20)
+    assert b.whats(res, qt, 640, k, m)[0] == "quantize tiled"  # the tiles and the tiled form's scratch
+    scratch = b.dev.scratch_device_bytes()
+    b.raw.fake_hip_limit(b.stat(LIVE))
+    freed, synced, refused = b.stat(FREES), b.stat(SYNCS), b.stat(REFUSED)
+    for _ in range(3):
+        assert b.whats(res, qt, rows, k, m) == ["quantize tiled", "gemm"]
+        assert b.dev.last_error() == ""
+    assert (b.stat(FREES), b.stat(SYNCS)) == (freed, synced)
+    assert b.stat(REFUSED) == refused + 1  # asked once
+    assert b.dev.scratch_device_bytes() == scratch
+    # memory that this library gives back is a reason to ask again; here it is still too little
+    b.dev.dev_free(spare)
+    assert b.whats(res, qt, rows, k, m) == ["quantize tiled", "gemm"]
+    assert b.stat(REFUSED) == refused + 2
+    b.raw.fake_hip_limit(NO_LIMIT)
+    assert b.whats(res, qt, rows, k, m) == ["quantize tiled", "gemm"]
+    b.dev.free_resident(b.resident(qt, 32, k))
+    assert b.whats(res, qt, rows, k, m) == ["quantize tiled", "gemm wide"]
+    assert b.dev.scratch_device_bytes() > scratch
+    b.dev.free_resident(res)

@@ -240,6 +240,7 @@ struct zlm_device {
     // prefill scratch: quantized activations (qx, dx, sums) and staged x/out
     uint8_t* q_scratch = nullptr;
     uint64_t q_scratch_cap = 0;
+    uint64_t q_scratch_refused = UINT64_MAX;  // fewest bytes an optional growth was refused (grow_gemm_scratch)
     hipStream_t stream = nullptr;
 
     Slot slots[kRing];
@@ -480,6 +481,30 @@ bool ensure_bytes(zlm_device* d, uint8_t*& p, uint64_t& cap, uint64_t n) {
     cap = n;
     return true;
 }
+
+// Growth of the GEMM activation scratch for a call that also runs in what there
+// is: the larger buffer is allocated before the old one is given up, a refusal
+// leaves the scratch and the error text as they were, and the size is not asked
+// for again until this library gives device memory back (memory_given_back).
+bool grow_gemm_scratch(zlm_device* d, uint64_t n) {
+    if (n <= d->q_scratch_cap) return true;
+    if (d->capturing || d->gemm_graphs > 0 || n >= d->q_scratch_refused) return false;
+    uint8_t* p = nullptr;
+    if (hipMalloc(reinterpret_cast<void**>(&p), n) != hipSuccess) {
+        hipGetLastError();
+        d->q_scratch_refused = n;
+        return false;
+    }
+    if (d->q_scratch) {
+        hipStreamSynchronize(d->stream);
+        hipFree(d->q_scratch);
+    }
+    d->q_scratch = p;
+    d->q_scratch_cap = n;
+    return true;
+}
+
+void memory_given_back(zlm_device* d) { d->q_scratch_refused = UINT64_MAX; }
 
 // Every kernel launch of the library: the dispatch checked on the host
 // against what an AQL kernel-dispatch packet can carry (workgroup of 1..1024
@@ -1574,15 +1599,12 @@ bool enqueue_gemm(zlm_device* d, zlm_resident* r, uint32_t quant, size_t rows, s
     const uint64_t fbytes = mt * 32 * nb * 4;
     const uint64_t need = qbytes + fbytes * (with_min ? 2 : 1);
     // The wide kernel's activations: records of 128 tokens and two blocks, 1.4 times
-    // the tiled form's bytes.  Where the scratch holds the tiled form but cannot grow
-    // for the records (under capture, beside a graph that uses it, memory spent), or a
-    // launch could not cover them, the tiled kernels run.
+    // the tiled form's bytes.  Where the scratch cannot grow for the records (under
+    // capture, beside a graph that uses it, memory spent), or a launch could not cover
+    // them, the tiled kernels run.
     const uint64_t gt = (static_cast<uint64_t>(m) + 127) / 128, records = gt * ((nb + 1) / 2);
-    bool wide = !small && records < (1u << 21) && gemm_wide_pays(qi, rows, m, nb, d->cus, tiled_us);
-    if (wide && records * 14336 > d->q_scratch_cap) {
-        wide = !d->capturing && d->gemm_graphs == 0 && ensure_bytes(d, d->q_scratch, d->q_scratch_cap, records * 14336);
-        if (!wide) hipGetLastError();
-    }
+    const bool wide = !small && records < (1u << 21) && gemm_wide_pays(qi, rows, m, nb, d->cus, tiled_us) &&
+                      grow_gemm_scratch(d, records * 14336);
     if (need > d->q_scratch_cap && !may_replace_scratch(d, kUsesGemm, "the GEMM activation scratch")) return false;
     if (!ensure_bytes(d, d->q_scratch, d->q_scratch_cap, need)) return false;
     if (d->capturing) d->capture_uses |= kUsesGemm;
@@ -1735,6 +1757,7 @@ extern "C" zlm_resident* zlm_gpu_upload_resident(zlm_device* d, const void* byte
 extern "C" void zlm_gpu_free_resident(zlm_device* d, zlm_resident* r) {
     if (!r) return;
     if (d && d->avail) hipStreamSynchronize(d->stream);
+    if (d) memory_given_back(d);
     release_resident_memory(r);
     delete r;
 }
@@ -1766,6 +1789,7 @@ extern "C" bool zlm_gpu_release_gemm_tiles(zlm_device* d, zlm_resident* r) {
     if (!d || !d->avail || !r) return false;
     if (r->gemm_payload && !may_replace_scratch(d, kUsesGemm, "a resident's GEMM tiles")) return false;
     if (r->gemm_payload) hipStreamSynchronize(d->stream);
+    memory_given_back(d);
     free_gemm_tiles(r);
     return true;
 }
@@ -2410,6 +2434,7 @@ extern "C" void zlm_gpu_dev_free(zlm_device* d, void* p) {
     if (!d || !d->avail || !p) return;
     hipStreamSynchronize(d->stream);
     hipFree(p);
+    memory_given_back(d);
 }
 
 extern "C" bool zlm_gpu_dev_upload(zlm_device* d, void* dst, const void* src, size_t n) {
