@@ -412,10 +412,11 @@ bool zlm_gpu_attention_decode_enqueue_noalloc(zlm_device *dev, const float *qkv,
  * timers) fail while a capture is open.  Ops that allocate or convert layouts
  * on first use (a resident's first op, a resident's first matMul, the
  * attention and GEMM scratch) must have run once eagerly before their
- * capture; under capture they fail instead (a matMul of up to 8 tokens may
- * need neither tiles nor scratch and then builds none, so a wider one must
- * have run eagerly itself).  The library never frees or
- * replaces scratch that a captured graph references while that graph exists:
+ * capture; under capture they fail instead.  (An eager matMul of 5 to 8
+ * tokens prepares captures of up to 32 on its resident: where it ran without
+ * tiles and scratch, by a tall weight, zlm_gpu_capture_begin builds them; one
+ * of up to 4 tokens, and one of 5 to 8 that ran the int-path token GEMV,
+ * prepares none.)  The library never frees or replaces scratch that a captured graph references while that graph exists:
  * after capturing an attention call, an eager attention call that needs more
  * partials fails with the reason; after capturing a matMul, an eager matMul
  * that needs more activation scratch, a rebuild of a resident's GEMM tiles

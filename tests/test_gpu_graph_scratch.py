@@ -12,6 +12,7 @@ fresh device (so these calls size the scratch themselves):
   resident's GEMM tiles, replays checked against the eager result and the
   oracle's int path (oracle.matmul_int); a product whose wide form needs more
   scratch than its tiled form runs the tiled one where the scratch cannot grow;
+  eager tokens that ran the tall kernel, which builds neither, prepare a capture;
 * the host-buffer contract ops refuse to run under capture.
 """
 import math
@@ -232,6 +233,57 @@ def test_wide_gemm_falls_back_where_its_scratch_cannot_grow(fresh):
         assert whats() == ["gemm wide"]
         check()
         assert dev.scratch_device_bytes() > sized
+    finally:
+        dev.launch_log(False)
+        if graph is not None:
+            dev.graph_destroy(graph)
+        dev.dev_free(d_x)
+        dev.dev_free(d_o)
+        dev.free_resident(res)
+
+
+def test_capture_after_eager_tall_tokens(fresh):
+    """Eight eager tokens by a tall weight are followed by a capture of 20."""
+    dev = fresh
+    rows, k, m = 32768 + 33, 256, 20
+    q = zd.quant(zd.Q4_K)
+    w = synth.weights(synth.Q4_K, rows, k, seed=61)
+    x = synth.activation(62, m * k)
+    res = dev.upload_resident(w)
+    assert res is not None, dev.last_error()
+    d_x, d_o = dev.dev_malloc(x.nbytes), dev.dev_malloc(m * rows * 4)
+    dev.dev_upload(d_x, x)
+    graph = None
+
+    def out():
+        got = np.zeros(m * rows, np.float32)
+        dev.dev_download(got, d_o)
+        return got
+
+    try:
+        _say("graph scratch: eight tokens by a tall weight, eagerly, then twenty captured")
+        assert dev.mat_mul_enqueue(res, q, rows, k, 8, d_x, d_o), dev.last_error()
+        assert dev.launch_log(True)
+        assert dev.capture_begin(), dev.last_error()
+        try:
+            ok = dev.mat_mul_enqueue(res, q, rows, k, m, d_x, d_o)
+        finally:
+            graph = dev.capture_end()
+        assert ok and graph is not None, dev.last_error()
+        assert [r["what"] for r in dev.launch_log_read()] == ["tile weights", "quantize tiled", "gemm small"]
+        replays = []
+        for _ in range(3):
+            dev.dev_upload(d_o, np.full(m * rows, np.nan, np.float32))
+            dev.graph_launch(graph, 1)
+            replays.append(out())
+            assert dev.mat_mul_enqueue(res, q, rows, k, 5, d_x, d_o), dev.last_error()  # other work between
+            dev.sync()
+        assert dev.mat_mul_enqueue(res, q, rows, k, m, d_x, d_o), dev.last_error()
+        eager = out()
+        for got in replays:
+            np.testing.assert_array_equal(got.view(np.uint32), eager.view(np.uint32))
+        # f32 sums of 8 block terms
+        assert rel_l2(eager.reshape(m, rows), oracle.matmul_int(synth.Q4_K, w, k, rows, m, x)) <= 1e-6
     finally:
         dev.launch_log(False)
         if graph is not None:

@@ -114,3 +114,65 @@ def test_wide_gemm_where_memory_is_spent(box):
     assert b.whats(res, qt, rows, k, m) == ["quantize tiled", "gemm wide"]
     assert b.dev.scratch_device_bytes() > scratch
     b.dev.free_resident(res)
+
+
+# Eager 5 to 8 tokens by a tall weight are the whole preparation that a capture
+# of up to 32 tokens needs, as they are where the small-M GEMM runs them: the
+# tall kernel itself builds neither tiles nor scratch, so the capture's begin does.
+TALL = [(synth.Q4_0, 65536, 64), (synth.Q4_1, 32768, 4160), (synth.Q4_K, 32768, 256)]
+
+
+@pytest.mark.parametrize("qt,rows,k", TALL)
+def test_capture_after_eager_tall_tokens(box, qt, rows, k):
+    b = box(32 * k, 32 * rows)
+    res = b.resident(qt, rows, k)
+    assert b.whats(res, qt, rows, k, 8) == ["gemm tall"]
+    held = b.dev.resident_device_bytes(res)
+    assert held == zd.layout_bytes(zd.quant(qt), rows, k, False)  # no tiled copy yet
+    assert b.dev.capture_begin(), b.dev.last_error()
+    assert b.dev.resident_device_bytes(res) == zd.layout_bytes(zd.quant(qt), rows, k, True)
+    for m in (9, 32):
+        assert b.whats(res, qt, rows, k, m) == ["quantize tiled", "gemm small"]
+    assert b.whats(res, qt, rows, k, 8) == ["gemm tall"]
+    assert not b.run(res, qt, rows, k, 33)[0]  # more scratch than eight eager tokens ask for
+    assert "eager call before capture" in b.dev.last_error()
+    graph = b.dev.capture_end()
+    assert graph
+    b.dev.graph_destroy(graph)
+    mallocs = b.stat(MALLOCS)
+    assert b.dev.capture_begin()  # once is enough
+    b.dev.graph_destroy(b.dev.capture_end())
+    assert b.stat(MALLOCS) == mallocs
+    b.dev.free_resident(res)
+
+
+def test_capture_without_eager_tokens_is_refused(box):
+    qt, rows, k = TALL[0]
+    b = box(32 * k, 32 * rows)
+    few, released, freed = (b.resident(qt, rows, k) for _ in range(3))
+    assert b.whats(few, qt, rows, k, 4) == ["gemm tall"]  # 3 and 4 tokens never prepared a GEMM
+    for r in (released, freed):
+        assert b.whats(r, qt, rows, k, 8) == ["gemm tall"]
+    assert b.dev.release_gemm_tiles(released)
+    b.dev.free_resident(freed)
+    assert b.dev.capture_begin(), b.dev.last_error()
+    for r in (few, released):
+        assert not b.run(r, qt, rows, k, 16)[0]
+        assert "tiles must be built by an eager matMul" in b.dev.last_error()
+    b.dev.graph_destroy(b.dev.capture_end())
+    b.dev.free_resident(few)
+    b.dev.free_resident(released)
+
+
+def test_capture_begins_where_memory_for_the_tiles_is_spent(box):
+    qt, rows, k = TALL[0]
+    b = box(32 * k, 32 * rows)
+    res = b.resident(qt, rows, k)
+    assert b.whats(res, qt, rows, k, 8) == ["gemm tall"]
+    b.raw.fake_hip_limit(b.stat(LIVE))
+    assert b.dev.capture_begin()
+    assert b.dev.last_error() == ""
+    assert b.whats(res, qt, rows, k, 8) == ["gemm tall"]
+    assert not b.run(res, qt, rows, k, 16)[0]
+    b.dev.graph_destroy(b.dev.capture_end())
+    b.dev.free_resident(res)

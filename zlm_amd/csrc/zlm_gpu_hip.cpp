@@ -162,6 +162,7 @@ struct zlm_resident {
     void* gemm_scales = nullptr;  // f16 (q4_0, q8_0) or float2 (scale, min) (q4_1, q4_k)
     uint64_t gemm_nb = 0;
     uint64_t gemm_rt = 0;  // 32-row tiles
+    uint64_t tiles_due = 0;  // row length (blocks) whose tiles the next capture builds (build_tiles_due); 0 = none
     uint64_t layout_alloc = 0;  // device bytes of the layout allocation
     uint64_t gemm_alloc = 0;    // device bytes of the GEMM tile allocation
     zlm_device* owner = nullptr;
@@ -241,6 +242,7 @@ struct zlm_device {
     uint8_t* q_scratch = nullptr;
     uint64_t q_scratch_cap = 0;
     uint64_t q_scratch_refused = UINT64_MAX;  // fewest bytes an optional growth was refused (grow_gemm_scratch)
+    std::vector<zlm_resident*> tiles_due;  // the residents with tiles_due set
     hipStream_t stream = nullptr;
 
     Slot slots[kRing];
@@ -1475,6 +1477,12 @@ uint64_t gemm_tile_bytes(uint32_t type, uint64_t rows, uint64_t nb) {
     return rt * nb * 32 * (type == ZLM_GGML_Q8_0 ? 32 : 16) + rt * nb * 32 * (gemm_has_min(type) ? 8 : 2);
 }
 
+// Bytes of the GEMM's quantized activations: m tokens, padded to whole 32-token
+// tiles, of nb blocks (32 quants, a scale and for the min-carrying types a sum).
+uint64_t gemm_scratch_bytes(uint32_t type, uint64_t m, uint64_t nb) {
+    return (m + 31) / 32 * 32 * nb * (32 + (gemm_has_min(type) ? 8 : 4));
+}
+
 void free_gemm_tiles(zlm_resident* r) {
     if (r->gemm_payload) hipFree(r->gemm_payload);
     r->gemm_payload = nullptr;
@@ -1482,6 +1490,14 @@ void free_gemm_tiles(zlm_resident* r) {
     r->gemm_nb = 0;
     r->gemm_rt = 0;
     r->gemm_alloc = 0;
+}
+
+void forget_tiles_due(zlm_device* d, zlm_resident* r) {
+    if (r->tiles_due == 0) return;
+    r->tiles_due = 0;
+    auto& due = d->tiles_due;
+    const auto it = std::find(due.begin(), due.end(), r);
+    if (it != due.end()) due.erase(it);
 }
 
 bool ensure_gemm_tiles(zlm_device* d, zlm_resident* r, const QuantInfo* qi, uint64_t nb) {
@@ -1524,7 +1540,34 @@ bool ensure_gemm_tiles(zlm_device* d, zlm_resident* r, const QuantInfo* qi, uint
     r->gemm_scales = ts;
     r->gemm_nb = nb;
     r->gemm_rt = rt;
+    forget_tiles_due(d, r);
     return true;
+}
+
+// A capture can build nothing, so the eager matMul before it builds the tiles and
+// the activation scratch that it needs, for up to 32 tokens whatever the eager
+// call's own number.  The tall kernel needs neither; a resident that it ran 5 to 8
+// tokens of is noted here instead, and the next capture's begin prepares it, so
+// that only callers who capture hold the tiled copy.  What memory does not allow
+// is left out: a captured call that needs it fails with the reason, as it would
+// without an eager call.
+void note_tiles_due(zlm_device* d, zlm_resident* r, uint64_t nb) {
+    if (d->capturing || r->tiles_due == nb || (r->gemm_payload && r->gemm_nb == nb)) return;
+    if (r->tiles_due == 0) d->tiles_due.push_back(r);
+    r->tiles_due = nb;
+}
+
+void build_tiles_due(zlm_device* d) {
+    const std::string err = d->err;
+    while (!d->tiles_due.empty()) {
+        zlm_resident* r = d->tiles_due.back();
+        const uint64_t nb = r->tiles_due;
+        forget_tiles_due(d, r);
+        const QuantInfo* qi = quant_info(r->layout);
+        if (!grow_gemm_scratch(d, gemm_scratch_bytes(qi->type, kGemmSmallM, nb)) || !ensure_gemm_tiles(d, r, qi, nb))
+            hipGetLastError();
+    }
+    d->err = err;
 }
 
 // Enqueue the prefill GEMM out_dev[t*rows + r] over a resident Q4_0, Q8_0,
@@ -1582,7 +1625,10 @@ bool enqueue_gemm(zlm_device* d, zlm_resident* r, uint32_t quant, size_t rows, s
             if (!enqueue_gemv(d, r, quant, rows, k, x_dev + t * k, out_dev + t * rows)) return false;
         return true;
     }
-    if (gemm_tall_pays(qi, rows, k, m)) return enqueue_gemm_tall(d, r, qi, rows, k, m, x_dev, out_dev);
+    if (gemm_tall_pays(qi, rows, k, m)) {
+        if (m > kQ8TokM && !pick_q8tok8(d, qi, k, rows)) note_tiles_due(d, r, nb);
+        return enqueue_gemm_tall(d, r, qi, rows, k, m, x_dev, out_dev);
+    }
     {  // a few tokens: the int path in one pass over the GEMV layout, no tiled copy or quantizer launch
         bool ran = false;
         if (!enqueue_gemv_q8tok(d, r, qi, rows, k, m, x_dev, out_dev, &ran)) return false;
@@ -1597,7 +1643,7 @@ bool enqueue_gemm(zlm_device* d, zlm_resident* r, uint32_t quant, size_t rows, s
     const uint64_t mt = (static_cast<uint64_t>(m) + 31) / 32;
     const uint64_t qbytes = mt * 32 * k;  // a multiple of 1024
     const uint64_t fbytes = mt * 32 * nb * 4;
-    const uint64_t need = qbytes + fbytes * (with_min ? 2 : 1);
+    const uint64_t need = gemm_scratch_bytes(qi->type, m, nb);
     // The wide kernel's activations: records of 128 tokens and two blocks, 1.4 times
     // the tiled form's bytes.  Where the scratch cannot grow for the records (under
     // capture, beside a graph that uses it, memory spent), or a launch could not cover
@@ -1758,6 +1804,7 @@ extern "C" void zlm_gpu_free_resident(zlm_device* d, zlm_resident* r) {
     if (!r) return;
     if (d && d->avail) hipStreamSynchronize(d->stream);
     if (d) memory_given_back(d);
+    if (d) forget_tiles_due(d, r);
     release_resident_memory(r);
     delete r;
 }
@@ -1791,6 +1838,7 @@ extern "C" bool zlm_gpu_release_gemm_tiles(zlm_device* d, zlm_resident* r) {
     if (r->gemm_payload) hipStreamSynchronize(d->stream);
     memory_given_back(d);
     free_gemm_tiles(r);
+    forget_tiles_due(d, r);
     return true;
 }
 
@@ -2081,6 +2129,7 @@ extern "C" bool zlm_gpu_mat_mul_batch(zlm_device* d, uint32_t quant, const void*
     if (!convert_blocks(d, d->s_raw, nblk, qi, d->s_lay, &view.scales)) return false;
     view.payload = d->s_lay;
     const bool ran = zlm_gpu_mat_mul_resident(d, &view, quant, rows, k, m, x, x_len, out, out_len);
+    forget_tiles_due(d, &view);
     view.payload = nullptr;
     view.scales = nullptr;
     return ran;
@@ -2887,6 +2936,7 @@ bool profiler_in_process() {
 extern "C" bool zlm_gpu_capture_begin(zlm_device* d) {
     if (!d || !d->avail) return false;
     if (d->capturing) return fail(d, "already capturing");
+    build_tiles_due(d);
     if (!ok(d, hipStreamBeginCapture(d->stream, hipStreamCaptureModeRelaxed), "begin capture")) return false;
     d->capturing = true;
     d->capture_uses = 0;
