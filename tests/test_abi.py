@@ -169,6 +169,28 @@ def test_profiler_check_sees_later_loads(tmp_path):
     subprocess.run([sys.executable, "-c", code], check=True, cwd=os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
 
 
+def test_profiler_check_keeps_no_failed_read(tmp_path):
+    """A process map that could not be read (no file descriptor left) is no answer
+    to keep: the next check reads it again."""
+    import subprocess
+    import sys
+    src = tmp_path / "empty.c"
+    src.write_text("int zlm_empty;\n")
+    fake = tmp_path / "librocprofiler-sdk-empty.so"
+    subprocess.run(["gcc", "-shared", "-fPIC", str(src), "-o", str(fake)], check=True)
+    code = ("import _ctypes, os, resource\nfrom zlm_amd import device as zd\n"
+            "assert not zd.profiler_loaded()\n"
+            f"_ctypes.dlopen({str(fake)!r}, 0)\n"
+            "soft, hard = resource.getrlimit(resource.RLIMIT_NOFILE)\n"
+            "low = os.dup(0)\nos.close(low)\n"  # the lowest free descriptor
+            "resource.setrlimit(resource.RLIMIT_NOFILE, (low, hard))\n"
+            "blind = zd.profiler_loaded()\n"
+            "resource.setrlimit(resource.RLIMIT_NOFILE, (soft, hard))\n"
+            "assert not blind\n"
+            "assert zd.profiler_loaded()\n")
+    subprocess.run([sys.executable, "-c", code], check=True, cwd=os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
+
+
 def _kernel_args(path):
     """{kernel name: [sizes of its explicit arguments]} from a code object's
     metadata (the ROCm LLVM tools read the bundle and the ELF notes)."""

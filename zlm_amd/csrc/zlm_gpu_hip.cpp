@@ -2895,22 +2895,24 @@ struct zlm_graph {
 // the older librocprofiler64) is mapped into this process (maps_path: a
 // /proc/<pid>/maps-format file; null = this process's own).  The HIP runtime's
 // own librocprofiler-register and torch's roctracer/roctx are always mapped
-// and do not count.
-bool profiler_in_maps(const char* maps_path) {
+// and do not count.  1 or 0, or -1 where the file could not be read to its end.
+int profiler_in_maps(const char* maps_path) {
     FILE* f = fopen(maps_path ? maps_path : "/proc/self/maps", "r");
-    if (!f) return false;
+    if (!f) return -1;
     char line[4096];
     bool found = false;
     while (!found && fgets(line, sizeof line, f))
         found = strstr(line, "librocprofiler-sdk") != nullptr || strstr(line, "librocprofiler64") != nullptr;
+    const bool whole = !ferror(f);
     fclose(f);
-    return found;
+    return found ? 1 : whole ? 0 : -1;
 }
 
 // profiler_in_maps(nullptr), the maps read again only when the loader has added
 // or removed objects since: reading them costs 0.4 ms in a process with torch
 // loaded, most of a small model's step; the loader's counters (of all its
-// namespaces) cost 0.1 us.
+// namespaces) cost 0.1 us.  A map that could not be read counts as none for this
+// call and is read again at the next.
 bool profiler_in_process() {
     struct Counts {
         unsigned long long adds, subs;
@@ -2927,7 +2929,9 @@ bool profiler_in_process() {
     static bool found = false;
     std::lock_guard<std::mutex> lock(mu);
     if (now.adds == 0 || now.adds != seen.adds || now.subs != seen.subs) {
-        found = profiler_in_maps(nullptr);
+        const int read = profiler_in_maps(nullptr);
+        if (read < 0) return false;
+        found = read == 1;
         seen = now;
     }
     return found;
@@ -2974,7 +2978,7 @@ extern "C" zlm_graph* zlm_gpu_capture_end(zlm_device* d) {
 constexpr int kGraphsInFlight = 4;
 
 extern "C" bool zlm_gpu_profiler_loaded(const char* maps_path) {
-    return maps_path ? profiler_in_maps(maps_path) : profiler_in_process();
+    return maps_path ? profiler_in_maps(maps_path) == 1 : profiler_in_process();
 }
 
 extern "C" bool zlm_gpu_kernel_convention(const char* name, int32_t* role, bool* struct_args) {
