@@ -176,3 +176,19 @@ def test_capture_begins_where_memory_for_the_tiles_is_spent(box):
     assert not b.run(res, qt, rows, k, 16)[0]
     b.dev.graph_destroy(b.dev.capture_end())
     b.dev.free_resident(res)
+
+
+@pytest.mark.parametrize("qt,rows,k,m", [(synth.Q4_0, 64, 256, 16), (synth.Q4_K, 32768, 256, 8), (synth.Q8_0, 64, 64, 2)])
+def test_streamed_weight_leaves_nothing_behind(box, qt, rows, k, m):
+    """matMulBatch over a host weight: its tiled copy goes with the call."""
+    b = box(m * k, m * rows)
+    w = np.zeros(rows * synth.row_bytes(qt, k), np.uint8)
+    x, out = np.zeros(m * k, np.float32), np.zeros(m * rows, np.float32)
+    assert b.dev.mat_mul_batch(zd.quant(qt), w, rows, k, m, x, out), b.dev.last_error()
+    live = b.stat(LIVE)
+    for _ in range(3):
+        assert b.dev.mat_mul_batch(zd.quant(qt), w, rows, k, m, x, out), b.dev.last_error()
+    assert b.stat(LIVE) == live
+    assert b.dev.capture_begin()  # and nothing of it is prepared for a capture
+    b.dev.graph_destroy(b.dev.capture_end())
+    assert b.stat(LIVE) == live

@@ -2130,6 +2130,7 @@ extern "C" bool zlm_gpu_mat_mul_batch(zlm_device* d, uint32_t quant, const void*
     view.payload = d->s_lay;
     const bool ran = zlm_gpu_mat_mul_resident(d, &view, quant, rows, k, m, x, x_len, out, out_len);
     forget_tiles_due(d, &view);
+    free_gemm_tiles(&view);
     view.payload = nullptr;
     view.scales = nullptr;
     return ran;
