@@ -192,3 +192,39 @@ def test_streamed_weight_leaves_nothing_behind(box, qt, rows, k, m):
     assert b.dev.capture_begin()  # and nothing of it is prepared for a capture
     b.dev.graph_destroy(b.dev.capture_end())
     assert b.stat(LIVE) == live
+
+
+# How a host matMul's x and y cross, either side of each line: y stored by the
+# product into pinned memory ("direct") or copied by DMA, x by the copy kernel or
+# by DMA (q8_0, q4_0 / q4_1 and q4_k store at their own rates).
+CROSS = [  # quant, rows, k, m, y direct, x by the copy kernel
+    (synth.Q4_0, 40960, 2048, 1, True, True), (synth.Q4_0, 40961, 2048, 1, False, True),
+    (synth.Q4_0, 131072, 1024, 1, False, True), (synth.Q4_K, 131072, 2048, 1, False, True),
+    (synth.Q4_K, 65536, 3072, 1, True, True), (synth.Q8_0, 65536, 3072, 1, False, True),
+    (synth.Q8_0, 65536, 3840, 1, True, True), (synth.Q4_0, 262145, 3072, 1, False, True),
+    (synth.Q4_0, 65536, 64, 2, True, True), (synth.Q4_0, 65537, 64, 2, False, True),
+    (synth.Q4_1, 131072, 64, 2, False, True), (synth.Q4_K, 131072, 256, 2, True, True),
+    (synth.Q4_K, 131073, 256, 2, False, True), (synth.Q8_0, 65537, 1024, 2, False, True),
+    (synth.Q8_0, 65537, 2048, 2, True, True),
+    (synth.Q8_0, 196608, 64, 4, True, True), (synth.Q8_0, 196609, 64, 4, False, True),
+    (synth.Q8_0, 49153, 4096, 4, True, True), (synth.Q4_1, 98305, 96, 8, False, True),
+    (synth.Q4_0, 131072, 64, 8, True, True), (synth.Q4_0, 131073, 64, 8, False, True),
+    (synth.Q4_0, 131073, 2048, 8, True, True),
+    (synth.Q4_0, 64, 4096, 56, True, True), (synth.Q4_0, 64, 4096, 57, True, False),
+    (synth.Q4_0, 98304, 32, 32, True, True), (synth.Q4_0, 98305, 32, 32, False, True),
+    (synth.Q4_0, 98305, 544, 32, False, False), (synth.Q4_0, 4096, 512, 500, False, False),  # the second tiled
+    (synth.Q4_K, 8192, 256, 64, False, True), (synth.Q4_K, 8192, 512, 64, False, False),
+]
+
+
+@pytest.mark.parametrize("qt,rows,k,m,direct,staged", CROSS)
+def test_host_matmul_crossing(box, qt, rows, k, m, direct, staged):
+    b = box(16, 16)
+    res = b.resident(qt, rows, k)
+    x, out = np.zeros(m * k, np.float32), np.zeros(m * rows, np.float32)
+    h2d, d2h = b.stat(H2D), b.stat(D2H)
+    assert b.dev.launch_log(True)
+    assert b.dev.mat_mul_resident(res, zd.quant(qt), rows, k, m, x, out), b.dev.last_error()
+    assert (b.stat(D2H) == d2h, b.stat(H2D) == h2d) == (direct, staged)
+    assert ("stage x" in [r["what"] for r in b.dev.launch_log_read()]) == staged
+    b.dev.free_resident(res)

@@ -1457,6 +1457,13 @@ bool gemm_wide_pays(const QuantInfo* qi, size_t rows, size_t m, size_t nb, int c
     return 8 * wgs >= 7 * n * c && 6.0 + 0.6 * static_cast<double>(n * nb) < tiled_us;
 }
 
+// Whether the split-K kernel runs the product; if not, *tiled_us is the tiled
+// kernels' prediction and *split their split.
+bool gemm_runs_small(const QuantInfo* qi, size_t rows, size_t m, size_t nb, int cus, double* tiled_us, int* split) {
+    *tiled_us = gemm_tiled_us(qi, rows, m, nb, cus, split);
+    return m <= kGemmSmallM || gemm_small_us(qi, rows, m, nb, cus) < *tiled_us;
+}
+
 bool gemm_supported(uint32_t type) {
     return type == ZLM_GGML_Q4_0 || type == ZLM_GGML_Q8_0 || type == ZLM_GGML_Q4_1 || type == ZLM_GGML_Q4_K;
 }
@@ -1638,8 +1645,8 @@ bool enqueue_gemm(zlm_device* d, zlm_resident* r, uint32_t quant, size_t rows, s
     if (r->gemm_rt * 32 < rows) return fail(d, "GEMM tiles too short");
     const bool with_min = gemm_has_min(qi->type);
     int split = 1;
-    const double tiled_us = gemm_tiled_us(qi, rows, m, nb, d->cus, &split);
-    const bool small = m <= kGemmSmallM || gemm_small_us(qi, rows, m, nb, d->cus) < tiled_us;
+    double tiled_us = 0.0;
+    const bool small = gemm_runs_small(qi, rows, m, nb, d->cus, &tiled_us, &split);
     const uint64_t mt = (static_cast<uint64_t>(m) + 31) / 32;
     const uint64_t qbytes = mt * 32 * k;  // a multiple of 1024
     const uint64_t fbytes = mt * 32 * nb * 4;
@@ -2073,16 +2080,42 @@ extern "C" bool zlm_gpu_mat_vec_resident_batch(zlm_device* d, size_t k, const fl
 // start and end (6 and 9 us), not by their bytes, so the copy kernel pulls x and the
 // product stores y straight into pinned host memory, as in the GEMV ops; large ones
 // by the bytes, which the DMA engine moves better.  Measured, us of the whole call,
-// DMA both ways and direct:
-//   q4_0 4096 x 4096 x 4 39 and 26, 12288 x 4096 x 8 60 and 46, 12288 x 4096 x 2 44
-//   and 32; q4_k 12288 x 4096 x 24 124 and 105, 262144 x 3840 x 5 413 and 329.
-//   x by the copy kernel: 896 KiB 105 -> 104 (q8_0 4096 x 4096 x 56), 1 MiB 102 -> 104
-//   (q4_0 4096 x 16384 x 16), 3.1 MiB 655 -> 680 (12288 x 4096 x 200).
-//   y from the product: 9.4 MiB 660 -> 640 (q4_0 12288 x 4096 x 200), 11.4 MiB 800 ->
-//   735 (q8_0 20000 x 4096 x 150), 24 MiB 1620 -> 1643 (12288 x 4096 x 512).  From the
-//   one- and two-token GEMVs, whose waves store a few rows at a time: 0.5 MiB 96 -> 86
-//   (q4_k 65536 x 3840), 1.2 MiB 181 -> 187 (q4_0 151936 x 4096).
-constexpr size_t kMatMulStageBytes = 896u << 10, kMatMulDirectBytes = 12u << 20, kMatMulDirectGemvBytes = 1u << 20;
+// x and y by DMA and by kernel:
+//   both: q4_0 4096 x 4096 x 4 37 and 26, 12288 x 4096 x 8 61 and 47, 12288 x 4096 x 2
+//   44 and 33; q4_k 12288 x 4096 x 24 124 and 105, 262144 x 3840 x 5 435 and 347.
+//   x: 768 KiB 95 and 92 (q4_0 4096 x 4096 x 48, y by DMA), 1 MiB 122 and 124 (x 64),
+//   2 MiB 207 and 220 (x 128).  With y by DMA the copy kernel saves 0-5 us up to 64 KiB
+//   of x and nothing past it.
+// Where y's line lies depends on how the product's waves store it, few rows at a
+// time and the sooner the shorter the rows are (us by DMA and direct, x by kernel):
+//   one token: 32768 x 1024 41 and 37; 65536 x 2048 58 and 61, 131072 x 1024 q4_0 86
+//   and 99, q4_k 83 and 93; but with longer rows 131072 x 3072 82 and 74, 262144 x 3840
+//   q4_k 177 and 153 (q8_0 131072 x 3072 112 and 122, 262144 x 3840 241 and 224);
+//   two tokens: 65536 x 2048 74 and 71; q4_0 131072 x 1024 134 and 138, q8_0 105 and 106,
+//   but q8_0 131072 x 3072 148 and 142, and q4_k (four-row tiles) 126 and 118;
+//   the token GEMV: q8_0 131072 x 1024 x 4 168 and 159, 262144 x 1024 x 4 310 and 316;
+//   262144 x 4096 x 4 445 and 387;
+//   the tall kernel: q4_0 262144 x 1024 x 4 264 and 261, x 8 514 and 521, 262144 x 4096 x
+//   8 558 and 511;
+//   the small-M GEMM: 12288 x 4096 x 64 q4_0 240 and 226, 100000 x 1024 x 31 676 and
+//   659; 65536 x 4096 x 50 (12.5 MiB of y) 840 and 845;
+//   the tiled GEMMs: 0-3% less direct, and as much between runs of one form (megabytes
+//   of y out of the pinned buffer), so theirs goes by DMA.
+constexpr size_t kMatMulStageBytes = 896u << 10, kMatMulStageDmaBytes = 64u << 10;
+
+static bool mat_mul_direct(zlm_device* d, const QuantInfo* qi, size_t rows, size_t k, size_t m) {
+    if (!qi || !gemm_supported(qi->type)) return false;  // refused further down
+    const size_t kib = (m * rows * sizeof(float) + 1023) >> 10;
+    if (m == 1) return kib <= (k >= (qi->type == ZLM_GGML_Q8_0 ? 3840 : 3072) ? 1024 : 160);
+    if (m <= kGemmGemvM)
+        return kib <= (qi->type == ZLM_GGML_Q4_K || (qi->type == ZLM_GGML_Q8_0 && k >= 2048) ? 1024 : 512);
+    if (gemm_tall_pays(qi, rows, k, m)) return kib <= (k < 2048 ? 4096 : 12288);
+    if (m <= kQ8Tok8M && (m <= kQ8TokM ? pick_q8tok(d, qi, k, rows) : pick_q8tok8(d, qi, k, rows)))
+        return kib <= (k < 4096 ? 3072 : 12288);
+    double us;
+    int split;
+    return kib <= 12288 && gemm_runs_small(qi, rows, m, k / 32, d->cus, &us, &split);
+}
 
 extern "C" bool zlm_gpu_mat_mul_resident(zlm_device* d, zlm_resident* r, uint32_t quant, size_t rows, size_t k,
                                          size_t m, const float* x, size_t x_len, float* out, size_t out_len) {
@@ -2090,14 +2123,14 @@ extern "C" bool zlm_gpu_mat_mul_resident(zlm_device* d, zlm_resident* r, uint32_
     if (!x || !out || m == 0 || x_len != m * k || out_len < m * rows) return fail(d, "bad buffers");
     if (!ensure_pair(d, d->d_x, d->h_x, d->x_cap, m * k, d->h_x_dev)) return false;
     if (!ensure_pair(d, d->d_y, d->h_y, d->y_cap, m * rows, d->h_y_dev)) return false;
-    if (m * k * sizeof(float) <= kMatMulStageBytes) {
+    const bool direct = mat_mul_direct(d, quant_info(quant), rows, k, m);
+    if (m * k * sizeof(float) <= (direct ? kMatMulStageBytes : kMatMulStageDmaBytes)) {
         if (!stage_x_sync(d, x, m * k)) return false;
     } else {
         memcpy(d->h_x, x, m * k * sizeof(float));
         if (!ok(d, hipMemcpyAsync(d->d_x, d->h_x, m * k * sizeof(float), hipMemcpyHostToDevice, d->stream), "stage x"))
             return false;
     }
-    const bool direct = m * rows * sizeof(float) <= (m <= kGemmGemvM ? kMatMulDirectGemvBytes : kMatMulDirectBytes);
     if (!enqueue_gemm(d, r, quant, rows, k, m, d->d_x, direct ? d->h_y_dev : d->d_y)) {
         hipStreamSynchronize(d->stream);
         return false;
