@@ -238,9 +238,10 @@ def test_gemm_split_block_ranges(dev, qt, zq, case, rows, k, m, plain_what, min_
 # host picks it: at least 7/8 of the CUs of its rounds busy.  It walks block pairs
 # in turns of three stages (three buffers), so every remainder of the stages by
 # three, odd nb, a last row tile of one row and a last token tile of one
-# token; and two rounds of whole tiles (m = 896: exactly 7/8).
+# token; and two rounds of whole tiles (m = 896: exactly 7/8), at the shortest rows
+# that several rounds are taken for.
 WIDE = [(synth.Q4_1, zd.Q4_1, 56 * 192 + 1, k, 385) for k in (1536, 1568, 1632, 1664)] + \
-       [(synth.Q4_K, zd.Q4_K, 56 * 192 + 1, 1792, 511), (synth.Q4_K, zd.Q4_K, 12288, 1536, 896)]
+       [(synth.Q4_K, zd.Q4_K, 56 * 192 + 1, 1792, 511), (synth.Q4_K, zd.Q4_K, 12288, 3072, 896)]
 
 
 @pytest.mark.parametrize("qt,zq,rows,k,m", WIDE, ids=[f"{GEMM_QUANT_IDS[c[0]]}-{c[2]}x{c[3]}-m{c[4]}" for c in WIDE])
@@ -261,7 +262,7 @@ def test_gemm_wide(dev, qt, zq, rows, k, m):
         out = np.zeros(m * rows, np.float32)
         dev.dev_download(out, out_dev)
         got = out.reshape(m, rows)
-        # f32 sums of nb <= 56 block terms, each within a few roundings: well below 1e-6
+        # f32 sums of nb <= 96 block terms, each within a few roundings: well below 1e-6
         for r0, r1 in ((0, 64), (rows // 2, rows // 2 + 32), (rows - 48, rows)):
             want = oracle.matmul_int(qt, w[r0 * rb:r1 * rb], k, r1 - r0, m, xs)
             assert rel_l2(got[:, r0:r1], want) <= 1e-6, (r0, r1)

@@ -228,3 +228,17 @@ def test_host_matmul_crossing(box, qt, rows, k, m, direct, staged):
     assert (b.stat(D2H) == d2h, b.stat(H2D) == h2d) == (direct, staged)
     assert ("stage x" in [r["what"] for r in b.dev.launch_log_read()]) == staged
     b.dev.free_resident(res)
+
+
+# Where the wide fp6 GEMM runs: one round of its workgroups (128 tokens x 192 rows, 256
+# CUs), or several where rows have 96 blocks and the rounds are 7/8 full.
+@pytest.mark.parametrize("qt,rows,k,m,what", [
+    (synth.Q4_1, 56 * 192, 1536, 512, "gemm wide"), (synth.Q4_1, 55 * 192, 1536, 512, "gemm"),
+    (synth.Q4_1, 49152, 96 * 32 - 32, 256, "gemm"), (synth.Q4_1, 49152, 96 * 32, 256, "gemm wide"),
+    (synth.Q4_K, 12288, 2816, 1024, "gemm"), (synth.Q4_K, 12288, 3072, 1024, "gemm wide"),
+    (synth.Q4_K, 49152, 256, 1024, "gemm"), (synth.Q4_0, 12288, 3072, 1024, "gemm")])
+def test_wide_gemm_route(box, qt, rows, k, m, what):
+    b = box(16, 16)
+    res = b.resident(qt, rows, k)
+    assert b.whats(res, qt, rows, k, m) == ["quantize tiled", what]
+    b.dev.free_resident(res)

@@ -1439,21 +1439,33 @@ double gemm_tiled_us(const QuantInfo* qi, size_t rows, size_t m, size_t nb, int 
 
 // - The wide fp6 kernel (q4_1, q4_k): rounds of one 128-token x 192-row
 //   workgroup per CU, 6 us + 0.6 us per block and round with its quantizer
-//   (4.5 us of them at 512 tokens, which the tiled prediction leaves out).  Measured
-//   on q4_k, tiled and wide: 12288 x 4096 x 512 91 and 83 us, x 1999 340 and 317;
-//   15360 x 3840 x 384 84 and 76, x 1999 396 and 370.  It has no smaller tile for
-//   what is left over, so where its last round is emptier the tiled kernels take
-//   over (15360 x 3840 x 512, 320 workgroups: 107 and 139); the line is seven
-//   eighths of all rounds' CUs, the range it was measured on.
+//   (4.5 us of them at 512 tokens, which the tiled prediction leaves out).  It has no
+//   smaller tile for what is left over, so where its last round is emptier the tiled
+//   kernels take over (15360 x 3840 x 512, 320 workgroups: 107 and 139); the line is
+//   seven eighths of all rounds' CUs, the range it was measured on.
+//   What it gains depends on the clocks: a prefill is tens of milliseconds of
+//   products, whose steady clocks favour it, a product after a pause runs both forms
+//   faster and the tiled one more so.  Measured, tiled -> wide, steady (400 products on
+//   end) and one after a pause, us:
+//     one round (40 products on end): 12288 x 1536 x 512 45.5 -> 42.7, 45.6 -> 45.4;
+//     12288 x 4096 x 512 96 -> 92, 99 -> 98; 49152 x 4096 x 128 106 -> 92, 106 -> 96;
+//     several rounds: 24576 x 1024 x 2048 182 -> 183, 188 -> 207; 12288 x 1536 x 2048 134 ->
+//     133, 147 -> 155; 12288 x 2048 x 2048 175 -> 171, 190 -> 199; 12288 x 3072 x 2048 255 ->
+//     245, 274 -> 284; 24576 x 3072 x 512 131 -> 121, 143 -> 144; 15360 x 3840 x 1999 391 ->
+//     370, 404 -> 418; 12288 x 4096 x 1024 171 -> 161, 183 -> 186.
+//   So several rounds take it from kGemmWideRoundsNb blocks a row, where the steady gain
+//   (4-7%) outweighs the single product's loss (1-4%); below, it is the other way round
+//   (49152 x 256 x 896 loses 20% in either).
 //   Rows longer than kGemmWideMaxNb blocks keep to the other kernels (the wide
 //   kernel's offsets are 32-bit).
-constexpr uint64_t kGemmWideMaxNb = 1u << 18;
+constexpr uint64_t kGemmWideMaxNb = 1u << 18, kGemmWideRoundsNb = 96;
 
 bool gemm_wide_pays(const QuantInfo* qi, size_t rows, size_t m, size_t nb, int cus, double tiled_us) {
     if (!gemm_has_min(qi->type) || nb > kGemmWideMaxNb) return false;
     const uint64_t c = static_cast<uint64_t>(cus);
     const uint64_t wgs = static_cast<uint64_t>((rows + 191) / 192) * static_cast<uint64_t>((m + 127) / 128);
     const uint64_t n = (wgs + c - 1) / c;
+    if (n > 1 && nb < kGemmWideRoundsNb) return false;
     return 8 * wgs >= 7 * n * c && 6.0 + 0.6 * static_cast<double>(n * nb) < tiled_us;
 }
 
