@@ -242,3 +242,14 @@ def test_wide_gemm_route(box, qt, rows, k, m, what):
     res = b.resident(qt, rows, k)
     assert b.whats(res, qt, rows, k, m) == ["quantize tiled", what]
     b.dev.free_resident(res)
+
+
+@pytest.mark.parametrize("qt,rows,m", [(synth.Q4_K, 32768, 5), (synth.Q4_1, 40001, 8), (synth.Q4_0, 65536, 3)])
+def test_tall_kernel_covers_the_chip(box, qt, rows, m):
+    """One workgroup per CU, also where that leaves some of its 16 waves without a 16-row tile."""
+    b = box(16, 16)
+    res = b.resident(qt, rows, 256)
+    ok, log = b.run(res, qt, rows, 256, m)
+    assert ok, b.dev.last_error()
+    assert [(r["what"], r["grid_x"], r["block"]) for r in log] == [("gemm tall", 256, 1024)]
+    b.dev.free_resident(res)

@@ -1595,15 +1595,18 @@ void build_tiles_due(zlm_device* d) {
 // the min-carrying types), then the int8-MFMA GEMM over the tiled weights.
 // The tall kernel (16-row tiles of the GEMV layout, a wave each, one 16-wave
 // workgroup per CU; no tiled copy, no quantizer launch) runs m = 3..8 where there
-// are tiles enough for the chip's 4096 waves: a tile is one wave's, so a call takes
-// at least as long as a tile, 1.6 us per 256 elements.  Measured, before and with
-// it, us: q4_k m = 8 32768 x 4096 35 and 28, x 1024 15 and 11, 24576 x 3840 26 and
-// 28; q4_1 m = 8 32768 x 4096 36 and 32, 24576 x 3840 30 and 27, 16384 x 4096 23 and
-// 32; q4_0 m = 8 65536 x 4096 42 and 32, 49152 x 4096 33 and 32, 32768 x 4096 23 and
-// 31.  At m = 3 and 4 the int token GEMV is closer: q4_k 65536 x 4096 42 and 32,
-// 65536 x 8192 80 and 75, 32768 x 4096 25 and 28; q4_0 and q4_1 win only with short
-// rows (q4_0 262144 x 2048 69 and 64, 65536 x 2048 22 and 19; 151936 x 4096 73 and 76,
-// 65536 x 8192 63 and 68).  k % 64: q4_0 and q4_1 scales are loaded in pairs.
+// are at least eight tiles a CU: a tile is one wave's, so a call takes at least as
+// long as a tile, 1.6 us per 256 elements.  Measured, the route before it and it, us:
+//   m = 5 to 8: q4_k 32768 x 1024 15 and 10, x 4096 36 and 21, x 8192 72 and 49; q4_1
+//   32768 x 4096 37 and 23, x 8192 73 and 51; q4_0 65536 x 4096 42 and 33, x 8192 95 and
+//   73.  Fewer rows stay where they were: it still gains there (q4_k and q4_1 16384 x
+//   4096 23 and 17, 22 and 20; q4_0 32768 x 4096 30 and 24), until a CU has two to four
+//   tiles (8192 x 4096 q4_k 16 and 17, q4_1 15 and 19; q4_0 16384 x 4096 14 and 17).
+//   m = 3 and 4, where the int token GEMV is closer: q4_k 65536 x 4096 42 and 32, 65536 x
+//   8192 80 and 75, 32768 x 8192 46 and 50; q4_0 and q4_1 win only with short rows (q4_0
+//   262144 x 2048 69 and 64, 65536 x 2048 22 and 19; 151936 x 4096 73 and 76, 65536 x 8192
+//   63 and 68).
+// k % 64: q4_0 and q4_1 scales are loaded in pairs.
 bool gemm_tall_pays(const QuantInfo* qi, size_t rows, size_t k, size_t m) {
     if (!gemm_tall_type(qi->type) || m < 3 || m > 8 || k > 8192 || k % 64) return false;
     if (m <= 4) return rows >= 65536 && (qi->type == ZLM_GGML_Q4_K || k <= 2048);
@@ -1616,8 +1619,9 @@ bool enqueue_gemm_tall(zlm_device* d, zlm_resident* r, const QuantInfo* qi, size
     const uint16_t* s = r->scales;
     uint32_t rows32 = static_cast<uint32_t>(rows), m32 = static_cast<uint32_t>(m), nb32 = static_cast<uint32_t>(k / 32);
     void* args[] = {&w, &s, const_cast<float**>(&x_dev), &out_dev, &rows32, &m32, &nb32};
-    const uint64_t wgs = (static_cast<uint64_t>(rows) + 255) / 256;  // 16 tiles of 16 rows each
-    const unsigned grid = static_cast<unsigned>(std::min<uint64_t>(wgs, static_cast<uint64_t>(d->cus)));
+    // tiles are dealt to the workgroups first and to their waves second
+    const uint64_t tiles = (static_cast<uint64_t>(rows) + 15) / 16;
+    const unsigned grid = static_cast<unsigned>(std::min<uint64_t>(tiles, static_cast<uint64_t>(d->cus)));
     return launch(d, d->gemm_tall[qi->slot][k <= 4096 ? 0 : 1], grid, 1024, args, "gemm tall");
 }
 
