@@ -218,11 +218,13 @@ int zlm_gpu_cu_count(const zlm_device *dev);
  * both copies. */
 bool zlm_gpu_vram_info(zlm_device *dev, uint64_t *free_bytes, uint64_t *total_bytes);
 /* HBM a resident holds now: its raw bytes until the first op converts them,
- * then the device layout, plus the prefill GEMM's tiled copy once the tiled
- * GEMM has run on it (more than 4 tokens, or 3-4 tokens at k > 8192, k >
- * 16384 for Q4_1 / Q4_K; fewer tokens, and 5-8 tokens where the eight-slot
- * int-path GEMV runs and 3-8 tokens by a tall q4_0, q4_1 or q4_k weight (the
- * tall kernel: from 32768 rows up, k <= 8192), read the device layout). */
+ * then the device layout, plus the prefill GEMM's tiled copy once a GEMM over
+ * tiles has run on it.  Which calls run without the tiled copy is the library's
+ * choice by size (at present up to 2 tokens, 3-4 at k <= 8192, 16384 for Q4_1 /
+ * Q4_K, 5-8 where zlm_gpu_mat_mul_enqueue names the eight-slot form, and 3-8 by
+ * a tall weight), and a capture's begin builds it for tall weights that 5-8
+ * tokens ran on: budget a weight that takes matMuls of more than 2 tokens with
+ * it (zlm_gpu_layout_bytes, with_gemm). */
 uint64_t zlm_gpu_resident_device_bytes(const zlm_resident *res);
 /* HBM a rows x k weight of `quant` will hold once converted (its device
  * layout), plus its GEMM tiled copy when `with_gemm` (tensors the plan also
@@ -256,16 +258,26 @@ bool zlm_gpu_mat_vec_batch_enqueue(zlm_device *dev, zlm_resident *const *res, ui
 /* Enqueue the matrix product out_dev[t*rows + r] (x_dev: m x k fp32,
  * token-major) over a Q4_0, Q8_0, Q4_1 or Q4_K resident, by token count:
  * m = 1 the fp GEMV; m = 2 the two-token fp GEMV (k <= 16384, else a GEMV per
- * token); m = 3, 4 at k <= 8192 (16384 for Q4_1 / Q4_K) the int-path token GEMV (q8 activations
- * quantized in its prologue, the weights read once from the device layout),
- * and its eight-slot form at m = 5..8 for Q4_1 at k <= 4096 and Q4_K there up
- * to 8192 rows; otherwise the q8 activation quantizer, then an int8-MFMA GEMM over the
- * tiled copy (built on first use): up to 32 tokens the split-K small-M
- * kernel, past that the small-M kernel over several 32-token tiles or the
- * 128 x 64 tiled GEMM (each tile's blocks split over four or two wave
- * groups on small grids), whichever the library's cost model predicts faster for
- * (rows, k, m).  A token's results do not depend on the other tokens of the
- * call within one kernel. */
+ * token); from 3 tokens q8 activations and exact block dots:
+ * - m = 3..8 by a tall weight the tall kernel (int8 MFMA straight from the device
+ *   layout; k <= 8192, a multiple of 64): m = 5..8 from 32768 rows for Q4_1 and Q4_K
+ *   and 65536 for Q4_0, m = 3, 4 from 65536 rows for Q4_K, and for Q4_0 and Q4_1
+ *   with k <= 2048;
+ * - m = 3, 4 at k <= 8192 (16384 for Q4_1 / Q4_K) the int-path token GEMV (the
+ *   activations quantized in its prologue, the weights read once from the device
+ *   layout), and its eight-slot form at m = 5..8 for Q4_1 at k <= 4096 and Q4_K
+ *   there up to 8192 rows;
+ * - otherwise the activation quantizer, then an MFMA GEMM over the tiled copy
+ *   (built on first use): up to 32 tokens the split-K small-M kernel, past that
+ *   the small-M kernel over several 32-token tiles, the 128 x 64 tiled GEMM (each
+ *   tile's blocks split over four or two wave groups on small grids) or for Q4_1
+ *   and Q4_K the 128 x 192 wide GEMM, whichever the library's cost model predicts
+ *   faster for (rows, k, m).
+ * A token's results do not depend on the other tokens of the call within one
+ * kernel.  The wide GEMM needs 1.4 times the activation scratch of the tiled one;
+ * where the scratch cannot grow (under capture, beside a graph that uses it,
+ * memory spent) the tiled one runs, whose results differ in the last bits: a
+ * product repeats its own bits under capture if it ran eagerly before. */
 bool zlm_gpu_mat_mul_enqueue(zlm_device *dev, zlm_resident *res, uint32_t quant, size_t rows, size_t k, size_t m,
                              const float *x_dev, float *out_dev);
 /* Enqueue `iters` prefill GEMMs (quantizer + GEMM each), rotating over `n_res`

@@ -93,7 +93,7 @@ __device__ __forceinline__ v16f fp6_dot(const v8i a, const v8i w, int scale_a) {
 // blocks' scale matrices dx (x) dw (lanes 0-31 give the first block's vectors,
 // 32-63 the second's), 32 fmas, one K = 2 f32 product that adds the min terms, and
 // 16 adds to the sums.  (Straight into the sums, the fmas and the min product took
-// 347 us at 15360 x 3840 x 1999 instead of 370, but round three times a pair at the
+// 347 us at 15360 x 3840 x 1999 where this form took 370, but round three times a pair at the
 // sums' size: 2.8e-7 against 64 bits, where the int8 form has 2.1e-7 and this
 // 1.5e-7.)
 //
@@ -103,17 +103,22 @@ __device__ __forceinline__ v16f fp6_dot(const v8i a, const v8i w, int scale_a) {
 // way in (two lanes a row; each wave one row tile's block, shared by the four
 // waves of that tile).  Three buffers: in stage s the waves read s and write
 // s + 2, so one barrier a stage suffices; global loads run a stage further ahead,
-// in registers (two: 373 us).
+// in registers (two stages ahead took 373 us where this took 370).
 //
-// Bound: VALU issue (96 fmas and adds and 25 instructions to expand and store, a
-// wave and stage), the MFMAs behind them and the phases the barrier keeps in step.
-// Against the int8 form (gemm_tiles<Q4_K>), the quantizers included: 12288 x 4096
-// x 512 (a workgroup on every CU) 91 -> 83 us, x 1999 (four rounds) 340 -> 317,
-// 15360 x 3840 x 1999 396 -> 370.  Measured slower: the weights' stores behind the
-// second row tile's MFMAs instead of the first's (3%), the activations read through
-// L1 without LDS, four buffers and a barrier every second stage, eight waves with a
-// unit's MFMAs issued under the previous unit's fmas (two waves a SIMD hide less
-// than the pipelining gains).
+// Bound: VALU issue and the matrix pipe, one after the other.  A wave's stage has 116
+// VALU instructions (96 fmas and adds, the expansion and the stores: 464 cycles) and 8
+// MFMAs (384 cycles: the dots, the scale matrices and the min terms 128 each), and only
+// a tenth of the MFMA cycles run beside VALU ones: over 15360 x 3840 x 1999 the two make
+// up 729,000 of a SIMD's 826,000 active cycles.  The barrier keeps the three waves'
+// phases in step, and f32 MFMAs take as long as the fp6 ones for a fraction of the work.
+// Against the int8 form (gemm_tiles<Q4_K>), the quantizers included, in long runs of
+// products: 12288 x 4096 x 512 (a workgroup on every CU) 96 -> 92 us, 15360 x 3840 x 1999
+// (five rounds) 386 -> 366; a single product after a pause 99 -> 98 and 404 -> 418, the
+// int8 form gaining more from the higher clocks there.
+// Measured slower: the weights' stores behind the second row tile's MFMAs instead of the
+// first's (3%), the activations read through L1 without LDS, four buffers and a barrier
+// every second stage, eight waves with a unit's MFMAs issued under the previous unit's
+// fmas (two waves a SIMD hide less than the pipelining gains).
 constexpr int kFp6RowTiles = 6, kFp6Waves = 12, kFp6Units = 2;
 
 static_assert(2 * kFp6RowTiles == kFp6Waves, "a wave expands one row tile's block");
@@ -164,8 +169,9 @@ __device__ __forceinline__ void gemm_fp6(const uint8_t* __restrict__ wq, const u
     const uint32_t nst = (nb + 1) / 2;  // stages
 
     // The operands' buffers, bounded so that weights past the row's end are
-    // zeros, their scales among them (activations past it re-read the last stage).  LDS offsets are per-lane bases, fixed for
-    // the whole loop, plus constants (the stages are unrolled over the buffers).
+    // zeros, their scales among them (activations past it re-read the last stage).
+    // LDS offsets are per-lane bases, fixed for the whole loop, plus constants (the
+    // stages are unrolled over the buffers).
     // (The scalar offsets of stages past the end are held at the buffers' sizes:
     // the bounds check subtracts them from the size.)
     const __amdgpu_buffer_rsrc_t ra = gemm_rsrc(qx + static_cast<size_t>(by) * nst * kFp6Record, nst * kFp6Record);

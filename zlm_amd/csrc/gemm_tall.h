@@ -27,16 +27,18 @@ typedef float v4f __attribute__((ext_vector_type(4)));
 //
 // Bound: the payload's reads, 16 rows x 64 B an instruction (twice the cache lines
 // a contiguous 1 KiB touches): q4_k 262144 x 3840 x 8 runs at 4.5 TB/s, 130 us,
-// where the copy rate would give 97.  The small-M GEMM took 269 (its 32-token
+// where the rate of a large copy, 5.15 TB/s, would give 113 (VALU instructions fill
+// 56 us of it, the matrix pipe 6).  The small-M GEMM took 269 (its 32-token
 // products and their scaling are VALU work for 24 tokens that are not there, and
 // its workgroups drain at their ends); q4_0 151936 x 4096 x 8 121 -> 78, q4_1 142
 // (the token GEMV) -> 82.  What mattered: each scale is loaded by one lane and
 // handed on by a shuffle (each lane loading its own: 136 and 102 us for 130 and
-// 80 at q4_k 262144 x 3840 and 151936 x 4096), and loads without the streaming hint
-// (its lines are read in two halves: 152 us with it).  Three or four iterations in
-// flight instead of two change nothing there and cost 2 us at 32768 rows.  q8_0
-// gained nothing (246 -> 231, 81 -> 84 at 65536 x 5120) and stays with the small-M
-// GEMM.
+// 80 at q4_k 262144 x 3840 and 151936 x 4096), loads without the streaming hint
+// (its lines are read in two halves: 152 us with it), and tiles dealt to the CUs
+// before their waves (16 tiles a workgroup first: q4_k 32768 x 4096 x 8 28 us for
+// 21).  Three or four iterations in flight instead of two change nothing at
+// 262144 x 3840 and cost 2 us at 32768 rows.  q8_0 gained nothing (246 -> 231, 81 ->
+// 84 at 65536 x 5120) and stays with the small-M GEMM.
 template <int QT>
 struct Tall {
     static constexpr bool MIN = gemm_has_min(QT);

@@ -381,7 +381,6 @@ bool load_kernels(zlm_device* d) {
     return true;
 }
 
-// A device buffer and a pinned host buffer of `n` floats sharing one capacity.
 // A device buffer and a pinned host buffer of n floats, and the host
 // buffer's device-side address (kernels read or write it directly); all three
 // are replaced together when the buffer grows.
@@ -1309,7 +1308,6 @@ void release_resident_memory(zlm_resident* r) {
     r->gemm_rt = 0;
 }
 
-// Stage host x into the synchronous-op device buffer.
 // Copy n floats from a pinned host buffer (its device address `src`) into
 // device memory on the stream: the library's copy kernel reading the host
 // memory directly (one dependent launch; cheaper than a DMA copy at these
@@ -1326,6 +1324,7 @@ bool stage_in(zlm_device* d, float* dst, const float* src, const float* src_host
     return ok(d, hipMemcpyAsync(dst, src_host, n * sizeof(float), hipMemcpyHostToDevice, d->stream), "stage x");
 }
 
+// Stage host x into the synchronous-op device buffer.
 bool stage_x_sync(zlm_device* d, const float* x, size_t n) {
     if (!ensure_pair(d, d->d_x, d->h_x, d->x_cap, n, d->h_x_dev)) return false;
     memcpy(d->h_x, x, n * sizeof(float));
@@ -1377,22 +1376,23 @@ double now_ns() {
     return static_cast<double>(ts.tv_sec) * 1e9 + static_cast<double>(ts.tv_nsec);
 }
 
-// The quants with a prefill GEMM and whether their tiles carry a min term.
 // Matrix products by token count m: up to kGemmGemvM tokens the fp path (the
 // production GEMV's arithmetic, as zlm's CPU runs small batches through its fp
 // batched GEMV, reference form/single.zig:258-292; cheaper than the int path's
 // quantizer + GEMM there): one token the GEMV, two the two-token GEMV (one
 // pass over the weights, k <= 16384; beyond it one GEMV per token).  From 3
-// tokens the int path: 3-4 tokens the int-path token GEMV where it covers k;
-// up to one 32-token tile the split-K small-M int GEMM (zlm_gemm_small_*: 16
+// tokens the int path: 3-8 tokens by a tall weight the tall kernel
+// (gemm_tall_pays); 3-4 tokens the int-path token GEMV where it covers k; up
+// to one 32-token tile the split-K small-M int GEMM (zlm_gemm_small_*: 16
 // waves per workgroup for q4_0 / q8_0, 8 for q4_1 / q4_k; one workgroup per
 // 32-row x 32-token tile); beyond it whichever of that kernel and the
 // 128 x 64 tiled int GEMM (each tile's blocks split over four or two wave
 // groups, or not) the cost model below predicts faster, or for q4_1 / q4_k the
-// wide fp6 GEMM where its rounds fill the chip.
+// wide fp6 GEMM where its rounds fill the chip (gemm_wide_pays).
 constexpr size_t kGemmGemvM = 2;
 constexpr size_t kGemmSmallM = 32;
 
+// Whether the quant's tiles carry a min term.
 bool gemm_has_min(uint32_t type) { return type == ZLM_GGML_Q4_1 || type == ZLM_GGML_Q4_K; }
 
 // Predicted microseconds of the int GEMM kernels for rows x k x m, fitted to
@@ -1451,8 +1451,8 @@ double gemm_tiled_us(const QuantInfo* qi, size_t rows, size_t m, size_t nb, int 
 //     12288 x 4096 x 512 96 -> 92, 99 -> 98; 49152 x 4096 x 128 106 -> 92, 106 -> 96;
 //     several rounds: 24576 x 1024 x 2048 182 -> 183, 188 -> 207; 12288 x 1536 x 2048 134 ->
 //     133, 147 -> 155; 12288 x 2048 x 2048 175 -> 171, 190 -> 199; 12288 x 3072 x 2048 255 ->
-//     245, 274 -> 284; 24576 x 3072 x 512 131 -> 121, 143 -> 144; 15360 x 3840 x 1999 391 ->
-//     370, 404 -> 418; 12288 x 4096 x 1024 171 -> 161, 183 -> 186.
+//     245, 274 -> 284; 24576 x 3072 x 512 131 -> 121, 143 -> 144; 15360 x 3840 x 1999 386 ->
+//     366, 404 -> 418; 12288 x 4096 x 1024 171 -> 161, 183 -> 186.
 //   So several rounds take it from kGemmWideRoundsNb blocks a row, where the steady gain
 //   (4-7%) outweighs the single product's loss (1-4%); below, it is the other way round
 //   (49152 x 256 x 896 loses 20% in either).
@@ -1476,18 +1476,11 @@ bool gemm_runs_small(const QuantInfo* qi, size_t rows, size_t m, size_t nb, int 
     return m <= kGemmSmallM || gemm_small_us(qi, rows, m, nb, cus) < *tiled_us;
 }
 
+// The quants with a prefill GEMM.
 bool gemm_supported(uint32_t type) {
     return type == ZLM_GGML_Q4_0 || type == ZLM_GGML_Q8_0 || type == ZLM_GGML_Q4_1 || type == ZLM_GGML_Q4_K;
 }
 
-// Build (once per row length) the GEMM's tiled copy of a resident weight, over
-// all whole rows it holds, rows padded to 32; nb = 32-element blocks per row:
-//   q4_0 / q8_0  payload [rt][nb][32 rows][16 / 32 B] + f16 scales [rt][nb][32]
-//                (from the split layout);
-//   q4_1 / q4_k  payload [rt][nb][32 rows][16 B nibbles] + (scale, min) float2
-//                [rt][nb][32] (q4_1 from its split layout, q4_k from its
-//                qs payload and records).
-// The resident's layout type never changes, so nb keys the copy.
 // Bytes of the GEMM's tiled copy of a weight of `rows` rows and nb 32-element
 // blocks per row: per 32-row tile and block, 16 (nibbles) or 32 (q8_0) bytes a
 // row plus the row's scale (f16) or (scale, min) float pair.
@@ -1519,6 +1512,14 @@ void forget_tiles_due(zlm_device* d, zlm_resident* r) {
     if (it != due.end()) due.erase(it);
 }
 
+// Build (once per row length) the GEMM's tiled copy of a resident weight, over
+// all whole rows it holds, rows padded to 32; nb = 32-element blocks per row:
+//   q4_0 / q8_0  payload [rt][nb][32 rows][16 / 32 B] + f16 scales [rt][nb][32]
+//                (from the split layout);
+//   q4_1 / q4_k  payload [rt][nb][32 rows][16 B nibbles] + (scale, min) float2
+//                [rt][nb][32] (q4_1 from its split layout, q4_k from its
+//                qs payload and records).
+// The resident's layout type never changes, so nb keys the copy.
 bool ensure_gemm_tiles(zlm_device* d, zlm_resident* r, const QuantInfo* qi, uint64_t nb) {
     if (r->gemm_payload && r->gemm_nb == nb) return true;
     if (d->capturing) return fail(d, "a resident's GEMM tiles must be built by an eager matMul before capture");
@@ -1589,10 +1590,6 @@ void build_tiles_due(zlm_device* d) {
     d->err = err;
 }
 
-// Enqueue the prefill GEMM out_dev[t*rows + r] over a resident Q4_0, Q8_0,
-// Q4_1 or Q4_K weight and device activations x_dev (m x k, token-major):
-// quantize x to q8 blocks into the tiled device scratch (plus dx*sum(q) for
-// the min-carrying types), then the int8-MFMA GEMM over the tiled weights.
 // The tall kernel (16-row tiles of the GEMV layout, a wave each, one 16-wave
 // workgroup per CU; no tiled copy, no quantizer launch) runs m = 3..8 where there
 // are at least eight tiles a CU: a tile is one wave's, so a call takes at least as
@@ -1625,6 +1622,11 @@ bool enqueue_gemm_tall(zlm_device* d, zlm_resident* r, const QuantInfo* qi, size
     return launch(d, d->gemm_tall[qi->slot][k <= 4096 ? 0 : 1], grid, 1024, args, "gemm tall");
 }
 
+// Enqueue the matrix product out_dev[t*rows + r] over a resident Q4_0, Q8_0, Q4_1
+// or Q4_K weight and device activations x_dev (m x k, token-major): a few tokens
+// straight from the device layout, more by quantizing x to q8 blocks into the device
+// scratch (plus dx*sum(q) for the min-carrying types) and a GEMM over the tiled
+// weights.
 bool enqueue_gemm(zlm_device* d, zlm_resident* r, uint32_t quant, size_t rows, size_t k, size_t m,
                   const float* x_dev, float* out_dev) {
     if (!d || !d->avail) return fail(d, "device unavailable");

@@ -807,10 +807,12 @@ extern "C" __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_pe
 
 // Its activations (gemm_fp6.h): the tiled quantizer's arithmetic into a record per
 // 128 tokens and block pair: the blocks' q as fp6 hi and lo parts, dx, dx * sum q.
-// Bound by the reads of x (17 us at 1999 tokens x 4096).  The codes' fields interleave four threads' elements (fp6_expand's order: field 4q + c
-// from the thread of place c, its elements permuted), so the threads transpose
-// their codes in two exchanges, each then holding 24 bits of four fields, and
-// three of each four store a dword of the hi and one of the lo codes.
+// Bound by VALU issue (299 instructions a wave, 15 of the 18 us at 1999 tokens x
+// 3840; its 44 MB would take 9).  The codes' fields interleave four threads'
+// elements (fp6_expand's order: field 4q + c from the thread of place c, its
+// elements permuted), so the threads transpose their codes in two exchanges, each
+// then holding 24 bits of four fields, and three of each four store a dword of the
+// hi and one of the lo codes.
 extern "C" __global__ void __launch_bounds__(256)
     zlm_quantize_fp6_tiled(const float* __restrict__ x, uint8_t* __restrict__ qx, uint32_t m, uint32_t nb) {
     // slots (32 tokens x 2 blocks x 4 tiles per record), eight threads each; the
