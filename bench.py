@@ -1,7 +1,7 @@
 #!/usr/bin/env python3
 """Headline benchmark of the MI355X HIP backend for zlm's quantized GEMV path.
 
-A step is one pass of the configs[1] workload -- the Qwen3-8B FFN GEMVs in
+A step is one pass of the headline workload -- the Qwen3-8B FFN GEMVs in
 Q8_0 at batch 1: gate 12288x4096, up 12288x4096, down 4096x12288 -- over
 weights already resident in HBM and activations already on the device.  Every
 step reads a different copy of the three weights (>= 512 MiB in rotation), so
@@ -16,7 +16,8 @@ roofline object reports the dominant kernel (the k=4096 Q8_0 GEMV of gate/up),
 timed on its own after ~50 ms of untimed launches, median of three runs; the
 other configs likewise.  The CPU baseline is the oracle's restatement of zlm's
 production sweep on the same gate weight, on one thread per physical core (at
-most 16, the CPU share of one GPU) and on one thread; configs[4] and [2] get
+most 16, the CPU share of one GPU) and on one thread; the prefill GEMM and the
+decode step get
 CPU figures of their own in `extra`.
 
 Prints one JSON line.  --gpus N with N > 1 is refused: this backend runs on one
@@ -196,7 +197,7 @@ def cpu_baseline(g: Gemv, budget_s: float):
 
 
 def cpu_prefill_sample(w: np.ndarray, rows: int, k: int, budget_s: float):
-    """configs[4] on the CPU: zlm's int path (q8 activations, Q4_0 intBlock)
+    """The 512-token prefill GEMM on the CPU: zlm's int path (q8 activations, Q4_0 intBlock)
     at zlm's speed over a 64-token sample of the 512-token workload, all
     threads of the pool; rates scale per token."""
     import oracle
@@ -218,7 +219,7 @@ def upload_rate(dev) -> dict:
     each planned tensor from the mmap'd image): a 256 MiB Q4_0 weight from
     ordinary (pageable) host memory, as an mmap'd file page is, uploaded 8
     times into fresh residents (2 GiB); host wall time per upload, median of
-    the 8, and the configs[2] model's 4.57 GB at that rate."""
+    the 8, and the decode model's 4.57 GB at that rate."""
     from zlm_amd import decode as zdec
 
     nb = (256 << 20) // 18
@@ -292,7 +293,7 @@ def split_efficiency(dev, threads: int) -> dict:
 
 
 def cpu_decode_sample(cfg, budget_s: float):
-    """configs[2] on the CPU: one token's projection GEMVs (q;k;v, o, gate, up,
+    """The decode step on the CPU: one token's projection GEMVs (q;k;v, o, gate, up,
     down per layer, times the layer count, plus the Q8_0 lm_head) with zlm's
     production sweep at zlm's speed on the pool's threads.  Attention and the
     elementwise glue are not included (on the GPU they are ~20% of a token)."""
@@ -323,7 +324,7 @@ def cpu_decode_sample(cfg, budget_s: float):
 
 def sections(dev, args, want, extra):
     """The reported sections after the headline: the other configs' GEMVs, the
-    configs[4] GEMM, the small-M sweep and the configs[2] decode step (each
+    512-token GEMM, the small-M sweep and the 36-layer decode step (each
     runs when want(section) says so); results go into `extra`."""
     only = args.only
     # ---- the other GEMV configs (reported, not the headline) --------------------
@@ -374,7 +375,7 @@ def sections(dev, args, want, extra):
             g.free()
         extra["other_models_lm_heads"] = lm
 
-    # ---- configs[4]: prefill GEMM, Q4_0 12288x4096 x 512 tokens, int8 MFMA ---------
+    # ---- prefill GEMM, Q4_0 12288x4096 x 512 tokens, int8 MFMA ---------
     if want("gemm"):
         rows, k, m = 12288, 4096, 512
         w = synth.weights(synth.Q4_0, rows, k, 0x5A4C4D04)
@@ -446,7 +447,7 @@ def sections(dev, args, want, extra):
                          "GEMM, whichever the host's cost model predicts faster")
         extra["small_m_matmul"] = sweep
 
-    # ---- configs[2]: decode step of a Qwen3-8B-shaped Q4_0 model, batch 1 ----------
+    # ---- decode step of a Qwen3-8B-shaped Q4_0 model, batch 1 ----------
     cfg = None
     if want("decode"):
         from zlm_amd import decode as zdec
@@ -575,7 +576,7 @@ def main():
     ap.add_argument("--no-cpu", action="store_true", help="skip the CPU baseline")
     ap.add_argument("--quick", action="store_true", help="headline workload only")
     ap.add_argument("--cpu-seconds", type=float, default=16.0,
-                    help="CPU-baseline budget: half on the headline GEMV, a quarter each on configs[4] and [2]")
+                    help="CPU-baseline budget: half on the headline GEMV, a quarter each on the GEMM and the decode step")
     ap.add_argument("--decode-eager", type=int, default=0, metavar="N",
                     help="run N eager decode steps instead of timing graph replays (for kernel-trace profiling)")
     ap.add_argument("--decode-replays", type=int, default=30, metavar="N",
@@ -583,12 +584,12 @@ def main():
     ap.add_argument("--no-long-context", action="store_true",
                     help="skip the decode step at 8192 and 32768 cached positions")
     ap.add_argument("--no-small-m", action="store_true",
-                    help="skip the small-token-count matMul sweep (its GEMVs share kernels with configs[0]/[3])")
+                    help="skip the small-token-count matMul sweep (its GEMVs share kernels with the other sections)")
     ap.add_argument("--counters", action="store_true",
                     help="short warm-ups and few launches per shape, for rocprofv3 --pmc passes (not a timing run)")
     ap.add_argument("--only", choices=("roofline", "gemvs", "gemm", "smallm", "decode"), default=None,
-                    help="run one section for a profiler: the roofline kernel's timing (configs[1] gate/up), the "
-                         "other configs' GEMVs, the configs[4] GEMM, the small-token-count matMul sweep or the "
+                    help="run one section for a profiler: the roofline kernel's timing (Q8_0 gate/up), the "
+                         "other GEMVs, the 512-token GEMM, the small-token-count matMul sweep or the "
                          "decode step; no JSON line")
     ap.add_argument("--calibrate-copy", type=int, default=0, metavar="BYTES",
                     help="also run the library copy kernel 5x over BYTES (for HBM traffic counter calibration)")
@@ -621,7 +622,7 @@ def main():
     if only in ("gemvs", "gemm", "smallm", "decode"):
         return sections(dev, args, want, {})
 
-    # ---- headline: configs[1], Q8_0 Qwen3-8B FFN GEMVs ------------------------------
+    # ---- headline: Q8_0 Qwen3-8B FFN GEMVs ------------------------------
     step_w = 2 * synth.weight_bytes(synth.Q8_0, 12288, 4096) + synth.weight_bytes(synth.Q8_0, 4096, 12288)
     copies = max(1, math.ceil(MALL_DEFEAT_BYTES / step_w))
     log(f"C1: generating Q8_0 gate/up/down, {copies} resident copies each")
@@ -741,7 +742,7 @@ def main():
                       for n, v in cpu["published_shapes_1_thread"].items()))
         extra["upload_resident"] = upload_rate(dev)
         log(f"uploadResident: {extra['upload_resident']['GBps']} GB/s from pageable host memory "
-            f"(configs[2] weights in {extra['upload_resident']['configs2_upload_s']} s)")
+            f"(Qwen3-8B weights in {extra['upload_resident']['configs2_upload_s']} s)")
         extra["split_efficiency"] = split_efficiency(dev, cpu["cores"])
         log(f"split probe (GPU rows [0, m/2) + {cpu['cores']} CPU threads [m/2, m)): "
             f"{extra['split_efficiency']['split_us']} us against {extra['split_efficiency']['gpu_us']} us "

@@ -15,7 +15,7 @@ def pytest_configure(config):
 
 @pytest.fixture(scope="session")
 def dev():
-    """The HIP device.  On a GPU box it must be available: a GPU test never
+    """The HIP device.  Where there is a GPU it must be available: a GPU test never
     passes on a CPU fallback."""
     from zlm_amd.device import Device
 

@@ -2,12 +2,12 @@
 
 * The lm_head GEMVs (reference lmHeadRows,
   src/kernels/linear/matvec/form/single.zig:294-360) at their real sizes:
-  configs[2]'s Q8_0 151936 x 4096 and configs[3]'s Q6_K 262144 x 3840, the
+  a Q8_0 151936 x 4096 and a Q6_K 262144 x 3840, the
   plain contract op (host x in, host logits out) and the RMSNorm-fused device
   form the decode step uses, against the oracle's lmHeadRows restatement
   (relative L2 <= 1e-3).  These shapes take the tall instances the host picks
   from 65536 rows; a ragged 65573-row Q8_0 case covers the last partial tile.
-* The configs[2] decode step at Qwen3-8B dimensions (hidden 4096, 32 q / 8 kv
+* The decode step at Qwen3-8B dimensions (hidden 4096, 32 q / 8 kv
   heads of 128, FFN 12288, vocab 151936, Q4_0 projections, Q8_0 lm_head, fp16
   KV of 2048), two layers, caches holding a 2047-token history: the step at
   position 2047 (attention over all 2048 positions) eager, then a replay of
@@ -88,7 +88,7 @@ def test_lm_head_full_size_matches_oracle(dev, name, qt, rows, k):
         dev.free_resident(res)
 
 
-# configs[2] dimensions with two layers (the per-layer kernels are the same in
+# Qwen3-8B dimensions with two layers (the per-layer kernels are the same in
 # every layer; two layers also check that layer i+1 reads layer i's output).
 QWEN3_8B_2L = zdec.DecodeConfig(n_layers=2, hidden=4096, n_heads=32, n_kv_heads=8, head_dim=128, ffn=12288,
                                 vocab=151936, max_seq=2048)

@@ -8,7 +8,7 @@
   through positions 0, 1, 2 and 70 against the oracle's layer sequence
   (block.zig:20-41), eager and replayed from one captured HIP graph:
   logits relative L2 <= 1e-3;
-* the configs[2] model (Qwen3-8B shapes, weights synthesised in HBM): an eager
+* the full model (Qwen3-8B shapes, weights synthesised in HBM): an eager
   step and graph replays give bit-identical, finite logits.
 """
 import math
@@ -212,7 +212,7 @@ def test_tiny_decode_steps_match_oracle(dev):
 
 
 def test_qwen3_8b_step_matches_oracle_and_graph_replays_match_eager(dev):
-    """configs[2] at full size: weights synthesised in HBM, caches holding a
+    """Qwen3-8B at full size: weights synthesised in HBM, caches holding a
     2047-token history; the step at position 2047 (attention over 2048) against
     the oracle's 36-layer sequence over the same weights and caches (read back
     from HBM; the GEMVs through the oracle's pooled production sweep,

@@ -285,7 +285,7 @@ def test_gemm_wide(dev, qt, zq, rows, k, m):
 
 
 def test_gemm_config4_rows_subset(dev):
-    """configs[4] at full size (12288 x 4096 Q4_0 x 512 tokens); rows checked
+    """The 512-token prefill at full size (12288 x 4096 Q4_0); rows checked
     against the oracle on a slice of the weight (a GEMM row depends only on its
     own weight row)."""
     rows, k, m = 12288, 4096, 512
@@ -317,7 +317,7 @@ def test_gemm_unsupported_quants_fall_back(dev):
 
 
 def test_gemm_q4_k_c3_shape_rows_subset(dev):
-    """A configs[3]-shaped Q4_K prefill (15360 x 3840, 96 tokens): row slices
+    """A Q4_K prefill of a 3840-wide model (15360 x 3840, 96 tokens): row slices
     against the int oracle."""
     rows, k, m = 15360, 3840, 96
     _say("gemm q4_k 15360x3840 m=96")

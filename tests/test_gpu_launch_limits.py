@@ -7,9 +7,9 @@ work-items in x; at most 65536 workgroups in y and z; static LDS <= 160 KiB)
 and fails with the parameters otherwise.  Here the launch log records every
 launch of: one eager decode step of the small Qwen3-shaped model and of a
 two-layer model at Qwen3-8B dimensions (the same launches, per layer, as the
-36-layer configs[2] step; the reference's decode loop is
+36-layer Qwen3-8B step; the reference's decode loop is
 runtime/executor.zig:45-86), the same step while it is captured into a graph,
-the configs[4] prefill GEMM with its small-M and GEMV routes, and the attention
+the 512-token prefill GEMM with its small-M and GEMV routes, and the attention
 at a 40000-position cache (the wide merge).  Each record must sit within the
 limits, and the step's launch count must be 1 + 6 layers + 1.
 """

@@ -1399,7 +1399,7 @@ bool gemm_has_min(uint32_t type) { return type == ZLM_GGML_Q4_1 || type == ZLM_G
 // gfx950 measurements (256 CUs; 10 shapes, 3840-15360 rows, k 3840-15360,
 // m 33-512, weights rotated past the Infinity Cache).  On those 100 points
 // the picks below lose 3.7 us in all against the fastest kernel, 3.0 of it
-// at configs[4]'s shape (below).
+// at 12288 x 4096 x 512 (below).
 // - The small-M kernel: a fixed part plus a rate per (32-row tile, 32-token
 //   tile, 32-element block): 7 us + 0.15 ns (q4_0, q8_0), 6 us + 0.25 ns (the
 //   min-carrying q4_1, q4_k: 8-wave workgroups).
@@ -1408,7 +1408,7 @@ bool gemm_has_min(uint32_t type) { return type == ZLM_GGML_Q4_1 || type == ZLM_G
 //   c(n) us per block.  q4_0 / q8_0: split over four wave groups (*split =
 //   4, 16-wave workgroups, a quarter of the blocks per wave) at n = 1,
 //   c = 0.195; over two (*split = 2, 8-wave workgroups) at n = 2, c = 0.345;
-//   unsplit from n = 3, c = 0.19n (configs[4]: the two-way split measured
+//   unsplit from n = 3, c = 0.19n (12288 x 4096 x 512: the two-way split measured
 //   2-3% faster there but re-read 1.3x the HBM bytes).  q4_1 / q4_k: split
 //   over two at n = 1, c = 0.26 (one resident workgroup per CU: 159 VGPRs and
 //   64 KB of LDS; four groups do not fit); unsplit past that, c = 0.475 /

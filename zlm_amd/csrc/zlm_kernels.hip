@@ -720,7 +720,7 @@ __device__ __forceinline__ void gemm_tiles(const uint8_t* __restrict__ wq, const
 }
 
 // The unsplit tiled GEMMs, for grids of three or more workgroups per CU
-// (q4_0 / q8_0; configs[4] is one) or more than one (q4_1 / q4_k: nb is the
+// (q4_0 / q8_0; 12288 x 4096 x 512 is one) or more than one (q4_1 / q4_k: nb is the
 // row's 32-element block count, k/32 for both).  There the split form below
 // is no faster: its 8-wave workgroups run two per CU and re-read more of the
 // weight panels through L2.

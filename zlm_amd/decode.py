@@ -53,7 +53,7 @@ class DecodeConfig:
         return (self.n_heads + 2 * self.n_kv_heads) * self.head_dim
 
 
-# configs[2]: Qwen3-8B shapes, Q4_0 projections, Q8_0 lm_head, fp16 KV of 2048.
+# Qwen3-8B shapes, Q4_0 projections, Q8_0 lm_head, fp16 KV of 2048.
 QWEN3_8B = DecodeConfig(n_layers=36, hidden=4096, n_heads=32, n_kv_heads=8, head_dim=128, ffn=12288,
                         vocab=151936, max_seq=2048)
 
