@@ -17,8 +17,7 @@ timed on its own after ~50 ms of untimed launches, median of three runs; the
 other configs likewise.  The CPU baseline is the oracle's restatement of zlm's
 production sweep on the same gate weight, on one thread per physical core (at
 most 16, the CPU share of one GPU) and on one thread; the prefill GEMM and the
-decode step get
-CPU figures of their own in `extra`.
+decode step get CPU figures of their own in `extra`.
 
 Prints one JSON line.  --gpus N with N > 1 is refused: this backend runs on one
 GPU.
@@ -576,7 +575,8 @@ def main():
     ap.add_argument("--no-cpu", action="store_true", help="skip the CPU baseline")
     ap.add_argument("--quick", action="store_true", help="headline workload only")
     ap.add_argument("--cpu-seconds", type=float, default=16.0,
-                    help="CPU-baseline budget: half on the headline GEMV, a quarter each on the GEMM and the decode step")
+                    help="CPU-baseline budget: half on the headline GEMV, a quarter each on the GEMM and the "
+                         "decode step")
     ap.add_argument("--decode-eager", type=int, default=0, metavar="N",
                     help="run N eager decode steps instead of timing graph replays (for kernel-trace profiling)")
     ap.add_argument("--decode-replays", type=int, default=30, metavar="N",

@@ -1,10 +1,10 @@
 """GPU parity at the benchmark configurations' full dimensions.
 
 * The lm_head GEMVs (reference lmHeadRows,
-  src/kernels/linear/matvec/form/single.zig:294-360) at their real sizes:
-  a Q8_0 151936 x 4096 and a Q6_K 262144 x 3840, the
-  plain contract op (host x in, host logits out) and the RMSNorm-fused device
-  form the decode step uses, against the oracle's lmHeadRows restatement
+  src/kernels/linear/matvec/form/single.zig:294-360) at their real sizes: a
+  Q8_0 151936 x 4096 and a Q6_K 262144 x 3840, the plain contract op (host x
+  in, host logits out) and the RMSNorm-fused device form the decode step uses,
+  against the oracle's lmHeadRows restatement
   (relative L2 <= 1e-3).  These shapes take the tall instances the host picks
   from 65536 rows; a ragged 65573-row Q8_0 case covers the last partial tile.
 * The decode step at Qwen3-8B dimensions (hidden 4096, 32 q / 8 kv

@@ -234,6 +234,7 @@ def test_host_matmul_crossing(box, qt, rows, k, m, direct, staged):
 # CUs), or several where rows have 96 blocks and the rounds are 7/8 full.
 @pytest.mark.parametrize("qt,rows,k,m,what", [
     (synth.Q4_1, 56 * 192, 1536, 512, "gemm wide"), (synth.Q4_1, 55 * 192, 1536, 512, "gemm"),
+    (synth.Q4_1, 49152, 42 * 32, 128, "gemm"), (synth.Q4_1, 49152, 43 * 32, 128, "gemm wide"),  # the shortest rows
     (synth.Q4_1, 49152, 96 * 32 - 32, 256, "gemm"), (synth.Q4_1, 49152, 96 * 32, 256, "gemm wide"),
     (synth.Q4_K, 12288, 2816, 1024, "gemm"), (synth.Q4_K, 12288, 3072, 1024, "gemm wide"),
     (synth.Q4_K, 49152, 256, 1024, "gemm"), (synth.Q4_0, 12288, 3072, 1024, "gemm")])

@@ -142,7 +142,9 @@ __device__ __forceinline__ uint2 gemm_ld8(__amdgpu_buffer_rsrc_t r, uint32_t vof
 }
 
 // Offsets are 32-bit: the host sends rows of more than 2^18 blocks to the other
-// GEMMs (nst * 14336 and nb * 512 stay below 2^32).
+// GEMMs (nst * 14336 and nb * 512 stay below 2^32), and rows of fewer than 43, where
+// its cost model has the tiled kernels faster (the loads of stages past the end would
+// cover those too).
 __device__ __forceinline__ void gemm_fp6(const uint8_t* __restrict__ wq, const uint8_t* __restrict__ wsc,
                                          const uint8_t* __restrict__ qx, float* __restrict__ out, uint32_t rows,
                                          uint32_t m, uint32_t nb) {
